@@ -785,12 +785,14 @@ prefill_dma_kernel(PrefillArgs a) {
     }
     return [vt_addr, vo](auto jc, int dt) {
       // the transposing reads are issued as inline asm: the compiler's own
-      // form of them waits for every load-to-LDS in flight
+      // form of them waits for every load-to-LDS in flight.  lo is an
+      // early-clobber output: sharing the address register, the first read
+      // could return before the second had taken its address.
       constexpr int kOff = 32 * decltype(jc)::value * G::kRowBytes;
       const uint32_t addr = vt_addr + (dt < kVrd ? vo[dt] : vo[dt - kVrd] ^ 128u);
       u32x2 lo, hi;
       asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4"
-                   : "=v"(lo), "=v"(hi)
+                   : "=&v"(lo), "=v"(hi)
                    : "v"(addr), "n"(kOff), "n"(kOff + 16 * G::kRowBytes));
       return __builtin_bit_cast(f16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
     };

@@ -343,3 +343,41 @@ def test_prefill_attention_rising_scores(torch_cuda, D, kernel_path):
     K.paged_attention_prefill(p, w)
     torch.cuda.synchronize()
     assert_close_f16(out.cpu().numpy(), want, what="prefill rising scores")
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_prefill_attention_full_chip_repeats(torch_cuda, int8):
+    """D = 64 with every CU busy: a wave then often stalls between the two
+    transposing V reads of a fragment, which must not share the register that
+    the first returns into.  Three launches give the same bits, equal to fp32
+    torch attention."""
+    torch = torch_cuda
+    from redline_amd import kernels as K
+    hq, hkv, D, S, n, bs = 16, 4, 64, 6, 1536, 16
+    nblk = n // bs
+    g = torch.Generator(device="cuda").manual_seed(64)
+    cache = K.KVCache(1, S * nblk + 1, hkv, D, bs, K.KVDType.kINT8 if int8 else K.KVDType.kFP16)
+    for t in cache.tensors(0):
+        if t is not None and t.dtype == torch.int8:
+            t.copy_(torch.randint(-127, 128, t.shape, generator=g, device="cuda", dtype=torch.int8))
+        elif t is not None:
+            t.normal_(generator=g) if t.dtype == torch.float16 else t.uniform_(0.008, 0.018, generator=g)
+    bb = ra.BatchBuilder(S * n, S, S, nblk, bs, 1)
+    for i in range(S):
+        bb.add(np.zeros(n, np.int32), 0, n, None, np.arange(1 + i * nblk, 1 + (i + 1) * nblk, dtype=np.int32))
+    meta, shape, lay = bb.write()
+    d_meta = dev(torch, meta)
+    q = torch.randn((S * n, hq * D), generator=g, device="cuda").half()
+    got = [run_prefill(torch, K, q, hq * D, hq, D ** -0.5, cache.layer(0), d_meta[lay["block_tables"]:],
+                       nblk, d_meta[lay["positions"]:], d_meta, lay, shape, S * n, D) for _ in range(3)]
+    for i, o in enumerate(got[1:]):
+        assert np.array_equal(o.view(np.uint16), got[0].view(np.uint16)), f"launch {i + 1} differs"
+    k, v, ks, vs = cache.tensors(0)
+    rows = lambda t, s: (t.float() if s is None else (t.float() * s[..., None]).half().float())[  # noqa: E731
+        1 + (S - 1) * nblk:].transpose(1, 2).reshape(n, hkv, D)
+    k, v = rows(k, ks), rows(v, vs)
+    mask = torch.ones((n, n), device="cuda", dtype=torch.bool).triu(1)
+    for h in range(0, hq, 5):
+        s = (q[-n:, h * D:(h + 1) * D].float() @ k[:, h // (hq // hkv)].t().contiguous()) * D ** -0.5
+        want = torch.softmax(s.masked_fill(mask, float("-inf")), -1) @ v[:, h // (hq // hkv)].contiguous()
+        assert_close_f16(got[0][-n:, h * D:(h + 1) * D], want.cpu().numpy(), what=f"head {h}")
