@@ -25,6 +25,8 @@
 //
 // Kernels (the launch policy picks by m and shape; the kernels' own comments
 // give the details):
+//   * the streaming kernel (gemv_stream.hip; few rows, K too long for the
+//     K-slice kernel, groups of 32 and 64): 8 waves split K of one tile;
 //   * the pair kernel (m < 8): a workgroup stages x once in LDS, already
 //     permuted, with sum(x) per chunk and row taken during the staging, and
 //     each wave walks one 16-row tile over the full K with a ring of chunk
@@ -41,152 +43,16 @@
 // The pair and slab kernels walk K in x passes when x does not fit the LDS
 // budget (x re-staged per pass, accumulators kept).
 // The INT8 weight-only GEMV (gemv_w8a16) runs the K-slice decomposition too
-// (gemv_w8_kslice_kernel), or the pair kernel's INT8 form.
+// (gemv_w8_kslice_kernel), the streaming kernel or the pair kernel's INT8 form.
 #include <algorithm>
 #include <type_traits>
 #include <utility>
 
-#include "device.hpp"
-#include "redline_amd/rlk.h"
-#include "status.hpp"
+#include "gemv_common.hpp"
+#include "gemv_stream.hpp"
 
 namespace rlk {
 namespace {
-
-struct W4Args {
-  const uint16_t* x;  // activations of this launch, [m, k]
-  const uint8_t* w;
-  const uint16_t* scales;
-  const uint16_t* offsets;
-  const uint16_t* bias;
-  void* y;            // [m, y_ld]
-  int m;              // activation rows (1 .. 16 MT)
-  int n, k, group_size, groups, nchunks;
-  int cpp;            // K chunks per x pass (a multiple of K-split ways x ring depth);
-                      // K-slice kernel: 16-row tiles per workgroup
-  int npass;
-  int xstride;        // halves per staged x row
-  int slab_off;       // bytes from the end of x to the first chunk-pair slab;
-                      // K-slice kernel: bytes from the LDS base to the partial sums
-  int y_ld;
-  int gq_shift;       // pair kernel: log2(group_size / 128)
-  int gpp;            // pair kernel: quantisation groups per x pass
-};
-
-constexpr int kModeF16 = 0, kModeF32 = 1, kModeSwiglu = 2;
-constexpr int kSlabRow = 144;                // bytes per slab row: 128 code bytes + 16 pad
-constexpr int kSlabBytes = 16 * kSlabRow;    // one wave's chunk-pair slab
-
-// Codes of one lane for one chunk: 32 K (16 bytes) for 128-K chunks, 8 K
-// (4 bytes) for 32-K chunks.  Weights are read exactly once: non-temporal.
-template <int KC>
-__device__ __forceinline__ u32x4 load_codes(const uint8_t* p) {
-  if constexpr (KC == 128) {
-    return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-  } else {
-    u32x4 v = {__builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p)), 0u, 0u, 0u};
-    return v;
-  }
-}
-
-// A value the compiler must keep in a VGPR without knowing it (the empty asm
-// emits no instruction).  With the code magic opaque, (x & mask) | magic is
-// selected as one v_and_or_b32 (mask in an SGPR); with both operands known
-// constants the compiler splits it into AND + OR, because gfx9 VOP3
-// encodings take no literal.  Writing the op itself as inline asm would hide
-// it from the compiler's hazard recognizer, which must pad a VALU write of an
-// MFMA source operand.
-__device__ __forceinline__ uint32_t opaque(uint32_t v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t magic) {
-  return (x & mask) | magic;
-}
-
-// The 8 codes of a word (nibble e = code of K offset e) as fp16 values
-// 64 + q, in the order (q0, q4, q1, q5, q2, q6, q3, q7): a nibble placed in
-// mantissa bits 4..7 of 64.0 (0x5400) reads 64 + q exactly.  The bias of 64
-// is removed through the offset term (o - 64 s), computed once per group in
-// fp32; it keeps the MFMA sums within a small factor of the unbiased ones.
-__device__ __forceinline__ f16x8 codes_f16(uint32_t word, uint32_t magic) {
-  constexpr uint32_t kMask = 0x00F000F0u;
-  const u32x4 r = {and_or(word << 4, kMask, magic), and_or(word, kMask, magic),
-                   and_or(word >> 4, kMask, magic), and_or(word >> 8, kMask, magic)};
-  return __builtin_bit_cast(f16x8, r);
-}
-constexpr float kCodeBias = 64.0f;
-
-// The K-slice kernel's form: 5 VALU per 8 codes instead of 7.  Nibbles in
-// mantissa bits 0..3 of 1024.0 read 1024 + q, in bits 4..7 of 64.0 read
-// 64 + q, so the word needs one shift: (q0, q4) and (q2, q6) take magic
-// m1024, (q1, q5) and (q3, q7) m64 -- the same element order as codes_f16.
-// The biases leave through sum(x * kBias2) per chunk.  The larger bias costs
-// fp32 sum bits (the kernel's relative error grows from ~1.5e-6 to ~2e-5 at
-// k = 4096; the fp32-output bound is 1e-4).
-__device__ __forceinline__ f16x8 codes_f16_2m(uint32_t word, uint32_t m1024, uint32_t m64) {
-  const uint32_t w8 = word >> 8;
-  const u32x4 r = {and_or(word, 0x000F000Fu, m1024), and_or(word, 0x00F000F0u, m64),
-                   and_or(w8, 0x000F000Fu, m1024), and_or(w8, 0x00F000F0u, m64)};
-  return __builtin_bit_cast(f16x8, r);
-}
-// The bias of each element of codes_f16_2m's output.
-constexpr f16x8 kBias2 = {1024, 1024, 64, 64, 1024, 1024, 64, 64};
-
-// 8 consecutive activations permuted to the codes' order.
-__device__ __forceinline__ f16x8 x_perm(u32x4 v) {
-  const f16x8 h = __builtin_bit_cast(f16x8, v);
-  return __builtin_shufflevector(h, h, 0, 4, 1, 5, 2, 6, 3, 7);
-}
-
-// v / d for 0 <= v < 2^21 through a float reciprocal: (v + 1/2) / d lies at
-// least 1/(2d) away from an integer and the float error is below 2^-22 * v/d.
-__device__ __forceinline__ int quot(int v, float inv_d) {
-  return static_cast<int>((static_cast<float>(v) + 0.5f) * inv_d);
-}
-
-__device__ __forceinline__ float swap_adjacent_lanes(float v) {
-  // quad_perm (1, 0, 3, 2): each lane reads its odd/even neighbour
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF,
-                                                            0xF, false));
-}
-
-// Output of one 16x16 tile: lane (qd, r16) holds rows m = m0 + 4 qd + e of
-// weight row `row`.
-template <int MODE>
-__device__ __forceinline__ void store_tile(const W4Args& a, f32x4 v, int m0, int row, int r16) {
-  if constexpr (MODE == kModeSwiglu) {
-    // (gate, up) = rows (2i, 2i + 1) sit in lanes (r16, r16 + 1)
-    f32x4 up;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) up[e] = swap_adjacent_lanes(v[e]);
-    if ((r16 & 1) != 0 || row >= a.n) return;
-    uint16_t* y = static_cast<uint16_t*>(a.y) + row / 2;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (m0 + e >= a.m) break;
-      const float g = round_f16(v[e]);
-      const float u = round_f16(up[e]);
-      y[static_cast<size_t>(m0 + e) * a.y_ld] =
-          __builtin_bit_cast(uint16_t, static_cast<_Float16>(silu_f16(g) * u));
-    }
-  } else {
-    if (row >= a.n) return;
-    const float b =
-        a.bias != nullptr ? static_cast<float>(__builtin_bit_cast(_Float16, a.bias[row])) : 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (m0 + e >= a.m) break;
-      const size_t at = static_cast<size_t>(m0 + e) * a.y_ld + row;
-      if constexpr (MODE == kModeF32) {
-        static_cast<float*>(a.y)[at] = v[e] + b;
-      } else {
-        static_cast<uint16_t*>(a.y)[at] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v[e] + b));
-      }
-    }
-  }
-}
 
 // A workgroup owns `wr` 16-row weight tiles (wr row waves, a runtime value)
 // times S K-split ways: wave w takes row slot w % wr and K part w / wr.
@@ -198,17 +64,9 @@ __device__ __forceinline__ void store_tile(const W4Args& a, f32x4 v, int m0, int
 // lines; the MFMA layout itself allows only 16 rows x 64 bytes) and moved to
 // the MFMA layout through a private LDS slab of the wave.
 //
-// At most 8 waves per workgroup (about one workgroup per CU, so two waves per
-// SIMD): a wave may use up to 256 VGPRs, which pays for a deep ring of loads
-// in flight.
-constexpr int kMaxWaves = 8;
-// Word 3 of a buffer resource for raw byte-addressed loads (32-bit data
-// format, no swizzle), and the cache-policy operand of the buffer-load
-// builtins that marks a load non-temporal.
-constexpr int kBufferFlags = 0x00020000;
-constexpr int kNtLoad = 2;
-// Largest weight the pair kernel addresses through 32-bit buffer offsets.
-constexpr uint64_t kMaxBufferBytes = 0x7FFFFFFFu;
+// At most 8 waves per workgroup (kMaxWaves; about one workgroup per CU, so two
+// waves per SIMD): a wave may use up to 256 VGPRs, which pays for a deep ring
+// of loads in flight.
 
 template <int S, int P, int KC, int MT, int MODE, int PR = 1>
 __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w4_kernel(W4Args a) {
@@ -1114,10 +972,6 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
   }
 }
 
-// LDS a workgroup may take: the device allows 160 KiB per workgroup.
-constexpr size_t kLdsBudget = 160 * 1024;
-constexpr int kNoFit = 1;  // launch(): the policy's smallest x pass exceeds the LDS budget
-
 template <int S, int P, int KC, int MT, int MODE, int PR = 1>
 int launch(W4Args a, int wr_max, hipStream_t stream) {
   if (PR == 2 && a.nchunks % 2 != 0) return kNoFit;
@@ -1252,19 +1106,32 @@ int launch_kslice(W4Args a, hipStream_t stream) {
 }
 
 // Launch policies, selectable for tuning sweeps through RLK_TUNE_W4_CFG.
-// Entry 0, the default, is the K-slice kernel (4 chunks per slice, two
-// tiles' pairs in flight) from m = 8 on, and the pair kernel below m = 8 or
-// where the K-slice kernel does not fit (4 pairs in flight up to m = 8, 2
-// above); 9, 10 and 11 are the pair kernel with 2, 8 and 4 pairs at every m;
+// Entry 0, the default, is the streaming kernel for few rows, and for many the
+// K-slice kernel (4 chunks per slice, two tiles' pairs in flight) from m = 8 on,
+// and the pair kernel below m = 8 or where the K-slice kernel does not fit (4
+// pairs in flight up to m = 8, 2 above); 9, 10 and 11 are the pair kernel with 2, 8 and 4 pairs at every m;
 // 12-15 the K-slice kernel with (chunks per slice, tiles in flight) = (4, 1),
-// (4, 2), (2, 2), (2, 4); 8 is the slab kernel with 8
-// chunk pairs in flight; 1-7 are slab-kernel variants (K-split ways, slots in
+// (4, 2), (2, 2), (2, 4); 16 the streaming kernel (gemv_stream.hip); 8 is the
+// slab kernel with 8 chunk pairs in flight; 1-7 are slab-kernel variants (K-split ways, slots in
 // flight per wave, most row waves per workgroup, chunks per slot).  Shapes the
 // pair kernel does not take (an odd chunk count, group_size / 128 not a power
 // of two) use the slab kernel; 32-K chunks always use its single-chunk form.
+template <int MODE>
+int launch_stream(const W4Args& a, hipStream_t s) {
+  return launch_gemv_stream(
+      StreamCall{a.x, a.w, a.scales, a.offsets, a.bias, a.y, a.m, a.n, a.k, a.group_size, MODE, a.y_ld}, s);
+}
+
 template <int KC, int MT, int MODE>
 int launch_cfg(const W4Args& a, int cfg, hipStream_t s) {
   int st = kNoFit;
+  const int tiles = (a.n + 15) / 16, cus = compute_units();
+  // Groups of 32 and 64 need a scale per MFMA step: the streaming kernel's
+  // transposed codes against the slab kernel's 4-byte loads (k = 4096, groups of
+  // 32, m = 1 / 8 / 32: n = 4096 6.4 / 7.1 / 9.6 against 17.4 / 21.6 / 40.5 us;
+  // n = 28672 26.7 / 29.1 / 55 against 41 / 42 / 48, equal at m = 16).
+  if (cfg == 16 || (KC == 32 && cfg == 0 && (a.m <= 8 || tiles <= 4 * cus))) st = launch_stream<MODE>(a, s);
+  if (st != kNoFit) return st;
   if constexpr (KC == 128) {
     switch (cfg) {
       case 8: st = launch<1, 8, KC, MT, MODE, 2>(a, 8, s); break;
@@ -1283,13 +1150,24 @@ int launch_cfg(const W4Args& a, int cfg, hipStream_t s) {
       case 6: st = launch<1, 8, KC, MT, MODE, 2>(a, 4, s); break;
       case 7: st = launch<2, 8, KC, MT, MODE>(a, 4, s); break;
       default:
-        // measured at the Llama-3.1-8B gate_up shape: the pair kernel with 4
-        // pairs in flight below m = 8 (m = 4: 14.5-14.8 against 15.1-15.9 us);
-        // the K-slice kernel with two tiles' pairs in flight from m = 8 on,
-        // where staging x per workgroup and reading it back from LDS per chunk
-        // cost the most (m = 8: 15.2-15.3 against 15.4-15.6 us, m = 16:
-        // 15.5-15.7 against 17.3-17.5, m = 32: 20.2 against 25.7)
-        if (a.m >= 8) st = launch_kslice<4, 2, MT, MODE>(a, s);
+        // Few rows: the streaming kernel, whose 8 waves per tile keep the
+        // loads of a compute unit in flight where the pair kernel has one wave
+        // (k = 4096, n = 4096, m = 1 / 4: 5.5 / 6.1 against 8.4 / 11.4 us) and
+        // whose wait for x is shorter than the K-slice kernel's (m = 8 / 16 /
+        // 32: 5.9 / 7.1 / 8.8 against 7.8 / 7.8 / 10.3).  Up to two tiles per
+        // compute unit it also beats the pair kernel (n = 8192, k = 5120: 9.6
+        // against 10.9 at m = 1, 20.3 against 36.6 at m = 32); at three they
+        // are equal and beyond that re-reading x per tile costs it more (n =
+        // 28672, k = 4096, m = 1: 19 against 14.3).
+        // Many rows, measured at the Llama-3.1-8B gate_up shape: the pair
+        // kernel with 4 pairs in flight below m = 8 (m = 4: 14.5-14.8 against
+        // 15.1-15.9 us); the K-slice kernel with two tiles' pairs in flight from
+        // m = 8 on, where staging x per workgroup and reading it back from LDS
+        // per chunk cost the most (m = 8: 15.2-15.3 against 15.4-15.6 us, m =
+        // 16: 15.5-15.7 against 17.3-17.5, m = 32: 20.2 against 25.7)
+        if (tiles <= cus) st = launch_stream<MODE>(a, s);
+        if (st == kNoFit && a.m >= 8) st = launch_kslice<4, 2, MT, MODE>(a, s);
+        if (st == kNoFit && tiles <= 2 * cus) st = launch_stream<MODE>(a, s);
         if (st == kNoFit)
           st = a.m <= 8 ? launch_pairs<4, MT, MODE>(a, s) : launch_pairs<2, MT, MODE>(a, s);
         break;
@@ -1387,13 +1265,17 @@ int launch_kslice_w8(W4Args a, hipStream_t stream) {
 }
 
 // INT8 weight-only GEMV (gemv_weight_only.cu:64-93): the K-slice kernel with
-// one tile's lines in flight where it fits (rows in whole tiles, K a multiple
-// of 512 up to 4096: at the Llama-3.1-8B gate_up shape 23.2 / 23.4 / 23.6 /
-// 26.4 us at m = 1 / 8 / 16 / 32 against 25.0 / 25.7 / 26.5 / 30.7 for the
-// pair kernel, same run), else the pair kernel's INT8 form with P = 4 pairs
-// in flight (equal to or faster than 2 and 8).  RLK_TUNE_W8_CFG = 1, 2, 3
-// selects the pair kernel with P = 2, 4, 8, and 4, 5, 6 the K-slice kernel
-// with (lines per slice, tiles in flight) = (4, 1), (4, 2), (2, 2).
+// one tile's lines in flight where it fits (rows in whole tiles, K a multiple of 512 up to 4096: at
+// the Llama-3.1-8B gate_up shape 23.2 / 23.4 / 23.6 / 26.4 us at m = 1 / 8 /
+// 16 / 32 against 25.0 / 25.7 / 26.5 / 30.7 for the pair kernel, same run).
+// Other K: the streaming kernel up to two tiles per compute unit (n = k = 5120,
+// m = 1 / 8 / 32: 10.4 / 13.0 / 22.9 against 12.7 / 14.9 / 28.2 us; n = 3584,
+// k = 18944: 14-15 / 18-20 / 33 against 38.7 / 59 / 134; at n = 10240 16.2 /
+// 20.4 / 35 against 16.2 / 18.0 / 28.3), else the pair kernel's INT8 form with
+// P = 4 pairs in flight (equal to or faster than 2 and 8).  RLK_TUNE_W8_CFG =
+// 1, 2, 3 selects the pair kernel with P = 2, 4, 8, 4, 5, 6 the K-slice kernel
+// with (lines per slice, tiles in flight) = (4, 1), (4, 2), (2, 2), and 7 the
+// streaming kernel.
 template <int MT, int MODE>
 int dispatch_w8(const W4Args& a, hipStream_t s) {
   int st = kNoFit;
@@ -1404,7 +1286,11 @@ int dispatch_w8(const W4Args& a, hipStream_t s) {
     case 4: st = launch_kslice_w8<4, 1, MT, MODE>(a, s); break;
     case 5: st = launch_kslice_w8<4, 2, MT, MODE>(a, s); break;
     case 6: st = launch_kslice_w8<2, 2, MT, MODE>(a, s); break;
-    default: st = launch_kslice_w8<4, 1, MT, MODE>(a, s); break;
+    case 7: st = launch_stream<MODE>(a, s); break;
+    default:
+      st = launch_kslice_w8<4, 1, MT, MODE>(a, s);
+      if (st == kNoFit && (a.n + 15) / 16 <= 2 * compute_units()) st = launch_stream<MODE>(a, s);
+      break;
   }
   if (st == kNoFit) st = launch_pairs<4, MT, MODE, true>(a, s);
   return st;

@@ -237,3 +237,37 @@ def test_gemv_w4_deterministic_and_errors(torch_cuda):
     K.gemv_w4a16(dx, 0, dw, ds, do, g, None, n, k, y)  # m = 0: no-op
     torch.cuda.synchronize()
     assert not y.any()
+
+
+@pytest.mark.parametrize("n,k,g", [(2, 128, 128), (97, 128, 32), (4098, 384, 128), (1000, 1152, 384),
+                                   (4112, 640, 64), (514, 4224, 32), (48, 14336, 128)])
+@pytest.mark.parametrize("m", [1, 2, 3, 8, 9, 17, 32])
+def test_gemv_w4_stream_shapes(torch_cuda, n, k, g, m):
+    """The streaming kernel (8 waves split K of one tile; x and scales by
+    load-to-LDS): one step and many, an odd number of 128-K chunks, rows that
+    do not fill tiles (n = 4098: workgroups of 10 rows), groups of 32, 64 and
+    non-powers of two, every activation layout; scales at an address that is
+    only 2-byte aligned.  fp32 sums of codes 64 + q over K <= 14336: about 10
+    times the product's own rounding, 1e-5 of the largest output (fp32
+    epsilon 6e-8 x ~10 x sqrt(K) / 10); fp16 and SwiGLU at fp16 tolerance."""
+    torch = torch_cuda
+    from redline_amd import kernels as K
+    say(f"gemv_w4 stream n={n} k={k} g={g} m={m}")
+    rng = np.random.default_rng(n + k + m)
+    packed, s, o, _ = int4_linear(rng, n, k, g, dense=False)
+    x = randn_f16(rng, (m, k))
+    bias = randn_f16(rng, (n,), 0.1)
+    want = oracle.gemv_w4a16(x, packed, s, o, g, bias)
+    with tune_knob("RLK_TUNE_W4_CFG", 16):
+        got = run_gemv(torch, x, packed, s, o, g, bias, f32=True)
+        got16 = run_gemv(torch, x, packed, s, o, g, bias)
+        gated = run_swiglu(torch, x, packed, s, o, g) if n % 2 == 0 else None
+        ds, do = (dev(torch, np.concatenate([[0], a.reshape(-1)]).astype(np.float16))[1:] for a in (s, o))
+        y = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        K.gemv_w4a16(dev(torch, x), m, dev(torch, packed), ds, do, g, dev(torch, bias), n, k, y, True)
+        torch.cuda.synchronize()
+    assert rel_max_err(got, want) <= 1e-5
+    assert np.array_equal(got, y.cpu().numpy())
+    assert_close_f16(got16, want.astype(np.float16), what="stream fp16")
+    if gated is not None:
+        assert_close_f16(gated, oracle.gemv_w4a16_swiglu(x, packed, s, o, g), what="stream swiglu")

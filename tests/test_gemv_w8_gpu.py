@@ -153,3 +153,22 @@ def test_gemv_w8_deterministic_and_errors(torch_cuda):
     K.gemv_w8a16(dx, 0, dq, ds, None, n, k, y)  # m = 0: no-op
     torch.cuda.synchronize()
     assert not y.any()
+
+
+@pytest.mark.parametrize("cfg,n,k", [(7, 2, 128), (7, 97, 384), (7, 4098, 1152), (7, 48, 18944)])
+@pytest.mark.parametrize("m", [1, 4, 5, 9, 17, 32])
+def test_gemv_w8_stream_shapes(torch_cuda, cfg, n, k, m):
+    """The streaming kernel (8 waves split K of one tile, x by load-to-LDS) from
+    one step on, with rows that do not fill tiles.  fp32 with a bias at the reference's bound, and fp16."""
+    say(f"gemv_w8 stream cfg={cfg} n={n} k={k} m={m}")
+    rng = np.random.default_rng(n + k + m)
+    q = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    s = rng.uniform(0.001, 0.01, n).astype(np.float16)
+    bias = randn_f16(rng, (n,), 0.02)
+    x = randn_f16(rng, (m, k))
+    want = oracle.gemv_w8a16(x, q, s, bias)
+    with tune_knob("RLK_TUNE_W8_CFG", cfg):
+        got = run_w8(torch_cuda, x, q, s, bias, True)
+        got16 = run_w8(torch_cuda, x, q, s, bias, False)
+    assert rel_max_err(got, want) <= 1e-4
+    assert_close_f16(got16, want, what="w8 stream f16")
