@@ -861,7 +861,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
   const int r16 = lane & 15, qd = lane >> 4;
   const bool low = (lane & 8) == 0;
   const int T = a.cpp;  // tiles per workgroup, a multiple of U
-  const int ntiles = a.n / 16;
+  const int ntiles = (a.n + 15) / 16;
   const int tile0 = blockIdx.x * T;
   f32x4* red = reinterpret_cast<f32x4*>(lds);  // [T][nw][MT][64 lanes]
   const int kb = a.k;
@@ -871,16 +871,16 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
       kBufferFlags);
   const __amdgpu_buffer_rsrc_t none = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.w), 0, 0, kBufferFlags);
   const int pc0 = (low ? qd : 4 + qd) * 16, pc1 = (low ? 4 + qd : qd) * 16;
-  const int vo0 = (low ? r16 : r16 - 8) * kb + pc0;
-  const int vo1 = (low ? r16 + 8 : r16) * kb + pc1;
+  const int vo0 = (low ? r16 : r16 - 8) * kb, vo1 = (low ? r16 + 8 : r16) * kb;
   const int nq = T * CPW;  // (tile, line) steps of this wave
   u32x4 ring[P][2];
   auto fetch = [&](int s, int q) {
     const int t = tile0 + q / CPW;
     const __amdgpu_buffer_rsrc_t res = (q < nq && t < ntiles) ? wres : none;
     const int soff = t * 16 * kb + (l0 + q % CPW) * 128;
-    ring[s][0] = __builtin_amdgcn_raw_buffer_load_b128(res, vo0, soff, kNtLoad);
-    ring[s][1] = __builtin_amdgcn_raw_buffer_load_b128(res, vo1, soff, kNtLoad);
+    const int last = (a.n - 1 - t * 16) * kb;  // rows past n re-read the last one
+    ring[s][0] = __builtin_amdgcn_raw_buffer_load_b128(res, min(vo0, last) + pc0, soff, kNtLoad);
+    ring[s][1] = __builtin_amdgcn_raw_buffer_load_b128(res, min(vo1, last) + pc1, soff, kNtLoad);
   };
 
   // x of the slice in the A layout above, staged as in the INT4 kernel
@@ -962,7 +962,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
   for (int t = wave; t < T; t += nw) {
     const int row = (tile0 + t) * 16 + r16;
     if (tile0 + t >= ntiles) break;
-    const float sc = static_cast<float>(__builtin_bit_cast(_Float16, a.scales[row]));
+    const float sc = static_cast<float>(__builtin_bit_cast(_Float16, a.scales[min(row, a.n - 1)]));
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       f32x4 sum = red[((t * nw) * MT + mt) * kWave + lane];
@@ -971,6 +971,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
     }
   }
 }
+
 
 template <int S, int P, int KC, int MT, int MODE, int PR = 1>
 int launch(W4Args a, int wr_max, hipStream_t stream) {
@@ -1239,17 +1240,21 @@ int gemv_w4(const char* what, const uint16_t* x, int m, const uint8_t* w, const 
 // their partials would not fit the LDS budget.
 template <int CPW, int U, int MT, int MODE>
 int launch_kslice_w8(W4Args a, hipStream_t stream) {
-  if (a.n % 16 != 0 || a.k % (128 * CPW) != 0 || a.k / (128 * CPW) > kMaxWaves) return kNoFit;
+  if (a.k % (128 * CPW) != 0 || a.k / (128 * CPW) > kMaxWaves) return kNoFit;
   const int nw = a.k / (128 * CPW);
-  const int ntiles = a.n / 16;
+  const int ntiles = (a.n + 15) / 16;
   const int cus = compute_units();
   auto lds_for = [&](int t) {  // the partial sums, which double as the x staging rows
     return std::max(static_cast<size_t>(t) * nw * MT * kWave * sizeof(f32x4),
                     static_cast<size_t>(nw) * 16 * 272);
   };
-  int T = (ntiles + cus - 1) / cus;
-  T = (T + U - 1) / U * U;
-  while (T > U && lds_for(T) > kLdsBudget) T -= U;
+  // The tiles spread evenly over whole rounds of compute units (one workgroup
+  // each): 128256 rows are 2 rounds of 16 tiles, not 1.6 of 20 (k = 4096,
+  // m = 1: 85.6 against 102 us), and at m = 32 4 rounds of 8, not 3.1 of 10
+  // (103 against 120 us).
+  int T = 0;
+  for (int rounds = 1; T == 0 || (T > U && lds_for(T) > kLdsBudget); ++rounds)
+    T = ((ntiles + rounds * cus - 1) / (rounds * cus) + U - 1) / U * U;
   if (lds_for(T) > kLdsBudget) return kNoFit;
   a.cpp = T;
   const size_t lds = lds_for(T);
@@ -1265,7 +1270,7 @@ int launch_kslice_w8(W4Args a, hipStream_t stream) {
 }
 
 // INT8 weight-only GEMV (gemv_weight_only.cu:64-93): the K-slice kernel with
-// one tile's lines in flight where it fits (rows in whole tiles, K a multiple of 512 up to 4096: at
+// one tile's lines in flight where it fits (K a multiple of 512 up to 4096: at
 // the Llama-3.1-8B gate_up shape 23.2 / 23.4 / 23.6 / 26.4 us at m = 1 / 8 /
 // 16 / 32 against 25.0 / 25.7 / 26.5 / 30.7 for the pair kernel, same run).
 // Other K: the streaming kernel up to two tiles per compute unit (n = k = 5120,

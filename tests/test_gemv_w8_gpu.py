@@ -155,11 +155,13 @@ def test_gemv_w8_deterministic_and_errors(torch_cuda):
     assert not y.any()
 
 
-@pytest.mark.parametrize("cfg,n,k", [(7, 2, 128), (7, 97, 384), (7, 4098, 1152), (7, 48, 18944)])
+@pytest.mark.parametrize("cfg,n,k", [(7, 2, 128), (7, 97, 384), (7, 4098, 1152), (7, 48, 18944),
+                                     (4, 97, 512), (4, 12351, 1024)])
 @pytest.mark.parametrize("m", [1, 4, 5, 9, 17, 32])
-def test_gemv_w8_stream_shapes(torch_cuda, cfg, n, k, m):
+def test_gemv_w8_stream_and_row_tails(torch_cuda, cfg, n, k, m):
     """The streaming kernel (8 waves split K of one tile, x by load-to-LDS) from
-    one step on, with rows that do not fill tiles.  fp32 with a bias at the reference's bound, and fp16."""
+    one step on, with rows that do not fill tiles, and the K-slice kernel with
+    a partial last tile.  fp32 with a bias at the reference's bound, and fp16."""
     say(f"gemv_w8 stream cfg={cfg} n={n} k={k} m={m}")
     rng = np.random.default_rng(n + k + m)
     q = rng.integers(-128, 128, (n, k), dtype=np.int8)
