@@ -7,8 +7,11 @@
 // q_start .. q_start + q_len - 1; new token i sits at position
 // past + i = ctx_len - q_len + i and attends to positions [0, past + i].
 //
-// The mapping is wave64 and matrix-core first:
-//   * a workgroup of 4 waves takes (sequence, 64 or 128 query rows, head); a
+// Three kernels: the ping-pong kernel (grids that fill the chip), the
+// load-to-LDS kernel (small grids) and the register-staged kernel (block tables
+// and block sizes neither takes).  The mapping is wave64 and matrix-core first
+// (the details of the latter two; the ping-pong kernel has its own comment):
+//   * a workgroup of 4 or 8 waves takes (sequence, 64 .. 256 query rows, head); a
 //     wave owns 16 or 32 query rows and keeps their q in registers as MFMA B
 //     operands;
 //   * K and V tiles of 64 keys are staged once per workgroup in LDS (K
@@ -65,7 +68,19 @@ struct PrefillArgs {
   rlk_attention_params p;
   rlk_prefill_attention_work w;
   int scale16;  // INT8 scales stored as fp16 (extension)
+  // ping-pong kernel: query heads per kv head, its reciprocal, kv heads x split = gridDim.x
+  int grp, split;
+  float inv_grp, inv_hkv;
 };
+
+// v / d for 0 <= v < 2^21 through a float reciprocal: (v + 1/2) / d lies at
+// least 1/(2d) away from an integer and the float error is below 2^-22 * v/d.
+__device__ __forceinline__ int quot(int v, float inv_d) {
+  return static_cast<int>((static_cast<float>(v) + 0.5f) * inv_d);
+}
+__device__ __forceinline__ int uniform_quot(int v, float inv_d) {
+  return __builtin_amdgcn_readfirstlane(quot(v, inv_d));
+}
 
 template <int D, bool kInt8>
 struct PfTile {
@@ -864,6 +879,459 @@ prefill_dma_kernel(PrefillArgs a) {
   stt.store(p, q0, qi, q_len, h, qd);
 }
 
+// The ping-pong kernel: the default for power-of-two block sizes of at least 8.
+//
+// A workgroup takes 256 query rows of one kv head, a row being one (token,
+// query head of the group) pair with the head fastest: the K and V tiles are
+// read once for all G heads of the group, short prompts fill the rows, and the
+// rows of a workgroup span 256 / G positions, so its waves need nearly the same
+// keys.  A wave owns 32 rows.
+//
+// Per tile of 64 keys a wave has a vector phase Y (softmax) and a matrix phase X
+// (P . V of this tile, q . K of the next).  The two waves of a SIMD (wave w and
+// w + 4) run them half a tile apart, held there by a barrier after each phase:
+// while one has the matrix cores the other has the vector ALU.  With both units
+// in one phase for all waves (the kernel above) each stood idle for two thirds
+// of the time.
+//
+// A wave issues one instruction in about 5 clocks, so X is bound by its
+// instruction count unless the products are large: v_mfma_f32_32x32x16_f16 (32
+// products of 32 clocks where 16x16x32 takes 64 of 16).  S^T = K Q^T gives lane
+// (h, c) = (lane / 32, lane % 32) the keys 8 a + 4 h + e (a, e = 0..3) of each
+// 32-key half for query row c, so the softmax is per lane with one exchange
+// between the halves; O^T = V^T P^T takes the probabilities as they lie (16 keys
+// a step: a = 2 s, 2 s + 1), and gives lane (h, c) dims 8 a + 4 h + e of row c.
+//
+// A wave's part of tile t + 2 is complete in LDS at the end of its X(t), one
+// barrier before the other group reads it.  Its stage is that of tile t - 2
+// (INT8, four stages) or t - 3 (FP16, five: requested a tile earlier), whose last
+// reader is the other group's X(t - 2), done when this Y(t) begins.
+//   FP16: load-to-LDS of tile t + 3 in X(t).
+//   INT8: the codes (16 bytes of K and V a lane, 8 at D = 64) and the row's
+//     scales go to registers two tiles earlier; Y(t) dequantises tile t + 2 into
+//     its fp16 stage, fp16(float(code) * scale).
+// 16-byte chunk c of row r lies at c ^ kswz(r) in a K tile and c ^ vswz(r) in a V
+// tile: the 16 rows of a K read then take 16 different slots of 256 bytes, and
+// the 4 rows x 64 bytes that 32 lanes of a transposing V read take fill them.
+// The 4 or 8 rows of a wave's load lie in one cache block, so the block comes by
+// scalar load and the address from scalar arithmetic.
+//
+// Measured (us; the kernel above -> this one): Qwen2 heads, 4 x 4096 new tokens at
+// depths 0 .. 12288, FP16 2421 -> 1782; Llama-3.1-8B heads, 4 x 4096 tokens, FP16
+// 1085 -> 560, INT8 with fp16 scales 1406 -> 638; 24 ragged prompts of 17 .. 900
+// tokens 331 -> 168.
+enum PfKV { kPfFP16, kPfInt8F32, kPfInt8F16 };  // cache and scale type
+
+template <int D, bool kInt8>
+struct PfPP {
+  static constexpr int kWaves = 8, kThreads = 64 * kWaves;
+  static constexpr int kBQ = kWaves * 32;
+  static constexpr int kRowBytes = 2 * D;
+  static constexpr int kTileBytes = kBK * kRowBytes;
+  static constexpr int kStageBytes = 2 * kTileBytes;
+  // tiles in LDS: t - 1 .. t + 2, and (FP16) t + 3 in flight
+  static constexpr int kStages = kInt8 ? 4 : 5;
+  static constexpr int kLds = kStages * kStageBytes;
+  // rows of one wave load (1 KiB of fp16 rows; 8 rows of codes)
+  static constexpr int kRows = kInt8 ? 8 : 1024 / kRowBytes;
+  static constexpr int kPieces = kBK / (kWaves * kRows);  // K (and V) loads per wave and tile
+  static constexpr int kCacheRow = kInt8 ? D : 2 * D;
+  __device__ static int kswz(int r) { return D == 128 ? r & 15 : (r >> 1) & 7; }
+  __device__ static int vswz(int r) { return D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2; }
+};
+
+// LDS reads the compiler does not track (it would wait for every load-to-LDS
+// in flight); the caller waits.  The first output is early-clobber: the second
+// read's address must outlive it.
+template <int kOff, int kSecond>
+__device__ __forceinline__ u32x4 read_v(uint32_t addr) {
+  u32x2 l, h;
+  asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4"
+               : "=&v"(l), "=v"(h)
+               : "v"(addr), "n"(kOff), "n"(kOff + kSecond));
+  return u32x4{l[0], l[1], h[0], h[1]};
+}
+template <int kOff>
+__device__ __forceinline__ u32x4 read_k(uint32_t addr) {
+  u32x4 v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(kOff));
+  return v;
+}
+// 16 bytes a lane from src to dst (wave-uniform) + 16 lane.  (A function of its
+// own: with the builtin two lambdas deep the host pass drops the kernel's stub.)
+__device__ __forceinline__ void load_to_lds(const unsigned char* src, unsigned char* dst) {
+  __builtin_amdgcn_global_load_lds(src, (RLK_LDS void*)dst, 16, 0, 0);
+}
+// LDS instructions of fragments [from, to): two each for the first vf (V), one for K
+constexpr int lds_reads(int from, int to, int vf) {
+  int n = 0;
+  for (int i = from; i < to; ++i) n += i < vf ? 2 : 1;
+  return n;
+}
+template <int I, int N, class F>
+__device__ __forceinline__ void unroll_range(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    unroll_range<I + 1, N>(f);
+  }
+}
+
+template <int D, PfKV KV>
+__global__ __launch_bounds__(512, 2) void prefill_pp_kernel(PrefillArgs a) {
+  constexpr bool kInt8 = KV != kPfFP16;
+  using G = PfPP<D, kInt8>;
+  constexpr int kSteps = D / 16, kDims = D / 32;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char pf_lds[];
+
+  const rlk_attention_params& p = a.p;
+  const rlk_prefill_attention_work& w = a.w;
+  // Sequences in reverse dispatch order and their last query tiles (the most
+  // keys) first: in a chunked-prefill batch the later chunks usually sit deeper
+  // in their sequences, so the longest workgroups start first.  gridDim.x is a
+  // multiple of 8, so blockIdx.x picks the XCD: one kv head (and every
+  // gridDim.x / hkv-th query tile) of every sequence, which shares K and V in
+  // that XCD's L2 and gives each XCD the same work whatever the sequences'
+  // lengths.
+  const int hkv = p.kv.num_kv_heads, grp = a.grp;
+  const int sub = uniform_quot(blockIdx.x, a.inv_hkv), kvh = blockIdx.x - sub * hkv;
+  const int seq = w.seq_ids[gridDim.z - 1 - blockIdx.z];
+  const int q_len = w.q_len[seq];
+  const int nrows = q_len * grp;  // (token, head) rows of this kv head
+  const int tile0 = (nrows + G::kBQ - 1) / G::kBQ - 1;  // the last tile
+  const int qrow0 = (tile0 - static_cast<int>(blockIdx.y) * a.split - sub) * G::kBQ;
+  if (qrow0 < 0) return;  // workgroup-uniform
+  const int q0 = w.q_start[seq], past = w.ctx_len[seq] - q_len;
+  const int lbs = __builtin_ctz(p.kv.block_size), bs = 1 << lbs;
+  typedef const __attribute__((address_space(4))) int32_t* ConstInts;
+  const ConstInts table =
+      (ConstInts)(p.block_tables + static_cast<size_t>(seq) * p.max_blocks_per_seq);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c32 = lane & 31, half = lane >> 5;
+  const int wrow0 = qrow0 + wave * 32;  // first row of this wave
+  const int wrows = min(nrows - wrow0, 32);
+  const int tok0 = uniform_quot(wrow0, a.inv_grp);
+  const int kv_end = past + uniform_quot(min(qrow0 + G::kBQ, nrows) - 1, a.inv_grp) + 1;
+  const int ntiles = (kv_end + kBK - 1) / kBK;
+  // tiles this wave attends
+  const int wtiles = wrows > 0 ? (past + uniform_quot(wrow0 + wrows - 1, a.inv_grp)) / kBK + 1 : 0;
+  const int row = wrow0 + c32;
+  const bool valid = row < nrows;
+  const int tok = quot(row, a.inv_grp), head = kvh * grp + row - tok * grp;
+  // key 8 a + 4 half + e of the 32 at k0 is attended where 8 a + e <= lim0 - k0
+  const int lim0 = valid ? past + tok - 4 * half : -(1 << 30);
+  f16x8 qb[kSteps];  // dims 16 ks + 8 half .. + 7
+#pragma unroll
+  for (int ks = 0; ks < kSteps; ++ks) {
+    qb[ks] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (valid)
+      qb[ks] = __builtin_bit_cast(
+          f16x8, load16(p.q + static_cast<size_t>(q0 + tok) * p.q_stride + head * D + 16 * ks + 8 * half));
+  }
+
+  // ---- tile loads.  Row r of piece u of a tile: u * 8 kRows + wave * kRows + lrow
+  constexpr int kLanes = 64 / G::kRows;  // lanes of a row
+  const int lrow = lane / kLanes, lcol = lane % kLanes;
+  const int srow = wave * G::kRows + lrow;  // (rows 8 kRows apart share their swizzle)
+  const int kx = (lcol ^ G::kswz(srow)) << 4, vx = (lcol ^ G::vswz(srow)) << 4;
+  const uint32_t head_cells = static_cast<uint32_t>(kvh) << lbs, block_cells = static_cast<uint32_t>(hkv) << lbs;
+  // Rows past kv_end, and tiles past the last, load its last key again (finite,
+  // and masked out of every row).
+  auto piece_pos = [&](int tile, int u) {  // position of the piece's first row (uniform)
+    return min(tile * kBK + (u * 8 + wave) * G::kRows, (kv_end - 1) / G::kRows * G::kRows);
+  };
+  // the blocks of the next tile to be loaded, by scalar load a phase ahead
+  int next_blk[G::kPieces];
+  auto look_up = [&](int tile) {
+#pragma unroll
+    for (int u = 0; u < G::kPieces; ++u) next_blk[u] = table[piece_pos(tile, u) >> lbs];
+  };
+  // cache cell of the piece's first row, and this lane's row in the piece
+  auto piece = [&](int tile, int u, uint64_t& cell, int& r) {
+    const int pos = piece_pos(tile, u);
+    cell = static_cast<uint64_t>(static_cast<uint32_t>(next_blk[u])) * block_cells + (head_cells + (pos & (bs - 1)));
+    r = min(lrow, kv_end - 1 - pos);
+  };
+  // FP16: load j of a tile (piece j / 2, K then V), and the whole tile
+  uint64_t cell_of[G::kPieces];
+  int row_of[G::kPieces];
+  auto issue_part = [&](int tile, int j) {
+    const int u = j / 2;
+    unsigned char* dst = pf_lds + (tile % G::kStages) * G::kStageBytes + (wave + 8 * u) * 1024;
+    if (j % 2 == 0) {
+      piece(tile, u, cell_of[u], row_of[u]);
+      load_to_lds(static_cast<const unsigned char*>(p.kv.k) + cell_of[u] * G::kCacheRow +
+                      static_cast<uint32_t>(row_of[u] * G::kCacheRow + kx),
+                  dst);
+    } else {
+      load_to_lds(static_cast<const unsigned char*>(p.kv.v) + cell_of[u] * G::kCacheRow +
+                      static_cast<uint32_t>(row_of[u] * G::kCacheRow + vx),
+                  dst + G::kTileBytes);
+    }
+  };
+  auto issue = [&](int tile) {
+#pragma unroll
+    for (int j = 0; j < 2 * G::kPieces; ++j) issue_part(tile, j);
+  };
+  // INT8: a lane's D / 8 codes of one K and one V row, and the rows' scales
+  constexpr int kCodes = D / 8;  // bytes
+  using Codes = typename std::conditional<D == 128, u32x4, u32x2>::type;
+  using Scale = typename std::conditional<KV == kPfInt8F16, _Float16, float>::type;
+  struct Raw {
+    Codes k, v;
+    Scale ks, vs;
+  };
+  auto fetch = [&](int tile, Raw& raw) {
+    uint64_t cell;
+    int r;
+    piece(tile, 0, cell, r);
+    const uint32_t ro = r * D + lcol * kCodes;
+    raw.k = *reinterpret_cast<const Codes*>(static_cast<const unsigned char*>(p.kv.k) + cell * D + ro);
+    raw.v = *reinterpret_cast<const Codes*>(static_cast<const unsigned char*>(p.kv.v) + cell * D + ro);
+    raw.ks = (reinterpret_cast<const Scale*>(p.kv.k_scale) + cell)[static_cast<uint32_t>(r)];
+    raw.vs = (reinterpret_cast<const Scale*>(p.kv.v_scale) + cell)[static_cast<uint32_t>(r)];
+  };
+  // 8 codes (part h of the lane's) as fp16(float(code) * scale) into the image
+  auto dequant = [&](int tile, const Codes& c, Scale scale, bool isv, int h) {
+    unsigned char* img = pf_lds + (tile % G::kStages) * G::kStageBytes + (isv ? G::kTileBytes : 0);
+    const u32x2 c8 = {c[2 * h], c[2 * h + 1]};
+    f16x8 f;
+    if constexpr (KV == kPfInt8F16) {
+      // the product of two fp16 values rounded once, as through fp32 (18-bit
+      // products are exact there)
+      f = int8x8_to_f16(c8) * scale;
+    } else {
+      // (code + 128) * scale - 128 * scale in one rounding: float(code) * scale
+      const float off = -128.0f * scale;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t w = c8[i / 4] ^ 0x80808080u;
+        f[i] = static_cast<_Float16>(fmaf(static_cast<float>((w >> (8 * (i % 4))) & 0xFFu), scale, off));
+      }
+    }
+    *reinterpret_cast<f16x8*>(img + srow * G::kRowBytes +
+                              (((lcol * (kCodes / 8) + h) ^ (isv ? G::vswz(srow) : G::kswz(srow))) << 4)) = f;
+  };
+
+  // ---- the matrix phase.  Fragments 0 .. kVF - 1 are the tile's V (key step
+  // i / kDims, dim tile i % kDims), the rest the next tile's K (dim step
+  // (i - kVF) / 2, 32-key half (i - kVF) % 2).  kAhead fragments are requested
+  // ahead of use; LDS reads return in order, so a wait counts the reads issued
+  // later.
+  constexpr int kVF = 4 * kDims, kKF = 2 * kSteps, kAhead = 6;
+  const int tk = (lane & 15) >> 2, tm = lane & 3;
+  // the swizzles leave a fragment's address at fragment 0's XOR a constant
+  const int vrow = 4 * half + tk;
+  const uint32_t vrd = G::kTileBytes + vrow * G::kRowBytes +
+                       (((2 * ((lane >> 4) & 1) + (tm >> 1)) ^ G::vswz(vrow)) << 4) + ((tm & 1) << 3);
+  const uint32_t krd = c32 * G::kRowBytes + ((half ^ G::kswz(c32)) << 4);
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((RLK_LDS unsigned char*)pf_lds));
+  auto stage_base = [&](int tile) { return lds0 + static_cast<uint32_t>(tile % G::kStages) * G::kStageBytes; };
+  typedef float f32x16 __attribute__((ext_vector_type(16)));
+  f32x16 o[kDims], s[2];
+  f16x8 pb[4];
+#pragma unroll
+  for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+  float m_run = -FLT_MAX, l_run = 0.f;
+  const float c = p.scale * 1.44269504088896340736f;  // e^((s - m) scale) = 2^(s c - m c)
+
+  // fragments [kFrom, kTo); beside(i) runs after fragment i's product
+  auto products = [&](auto fromc, auto toc, int tile, auto beside) {
+    constexpr int kFrom = decltype(fromc)::value, kTo = decltype(toc)::value;
+    const uint32_t va = stage_base(tile) + vrd, ka = stage_base(tile + 1) + krd;
+    u32x4 frag[kAhead];
+    auto request = [&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      if constexpr (i < kVF) {
+        constexpr int dt = i % kDims, st = i / kDims;
+        frag[i % kAhead] = read_v<16 * st * G::kRowBytes, 8 * G::kRowBytes>(va ^ (dt << 6));
+      } else {
+        constexpr int ks = (i - kVF) / 2, kt = (i - kVF) % 2;
+        frag[i % kAhead] = read_k<32 * kt * G::kRowBytes>(ka ^ (ks << 5));
+      }
+    };
+    constexpr int kEarly = kFrom + kAhead < kTo ? kFrom + kAhead : kTo;
+    unroll_range<kFrom, kEarly>(request);
+    unroll_range<kFrom, kTo>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      constexpr int last = i + kAhead < kTo ? i + kAhead : kTo;  // fragments i + 1 .. last - 1 are requested
+      constexpr int later = lds_reads(i + 1, last, kVF);
+      static_assert(later < 16, "lgkmcnt holds 4 bits");
+      u32x4 f = frag[i % kAhead];
+      asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(f) : "n"(later));
+      const f16x8 h = __builtin_bit_cast(f16x8, f);
+      if constexpr (i < kVF) {
+        o[i % kDims] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h, pb[i / kDims], o[i % kDims], 0, 0, 0);
+      } else {
+        constexpr int ks = (i - kVF) / 2, kt = (i - kVF) % 2;
+        const f32x16 zero = {};
+        s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h, qb[ks], ks == 0 ? zero : s[kt], 0, 0, 0);
+      }
+      if constexpr (i + kAhead < kTo) request(std::integral_constant<int, i + kAhead>{});
+      beside(ic);
+    });
+  };
+  // Online softmax of the scores of a tile (as softmax_max and softmax_exp
+  // above, over 32 keys a lane)
+  auto softmax = [&](int tile) {
+    const int k0 = tile * kBK;
+    if (k0 + kBK - 1 > past + tok0 || wrows < 32) {  // uniform: some key is past some row
+      const int lim = lim0 - k0;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (32 * kt + 8 * (i / 4) + i % 4 > lim) s[kt][i] = -FLT_MAX;
+    }
+    float mt = -FLT_MAX;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mt = fmaxf(mt, s[kt][i]);
+    mt = rows_max<true>(mt);  // the row's other half
+    const float m_new = fmaxf(m_run, mt);
+    const bool grew = (m_new - m_run) * c > 8.f;  // first valid tile: always
+    if (__any(grew)) {
+      const float e = __builtin_amdgcn_exp2f((m_run - m_new) * c);
+      const float alpha = grew ? e : 1.f;
+      if (grew) m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < kDims; ++dt) o[dt] *= alpha;
+    }
+    const float mc = m_run * c;
+    float ts = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s[kt][i] = __builtin_amdgcn_exp2f(fmaf(s[kt][i], c, -mc));  // masked: 2^-huge = 0
+        ts += s[kt][i];
+      }
+    l_run += ts;
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pb[st][i] = static_cast<_Float16>(s[st / 2][8 * (st % 2) + i]);
+  };
+  // a barrier that drains nothing and that nothing crosses
+  auto barrier = []() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // ---- tiles 0 and 1, then the scores of tile 0
+  auto convert = [&](int tile, const Raw& r) {
+#pragma unroll
+    for (int h = 0; h < kCodes / 8; ++h) {
+      dequant(tile, r.k, r.ks, false, h);
+      dequant(tile, r.v, r.vs, true, h);
+    }
+  };
+  Raw raw[2];
+  if constexpr (kInt8) {
+    Raw first[2];
+    // (the blocks of all four tiles in one scalar round trip)
+    int blk[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) blk[i] = table[piece_pos(i, 0) >> lbs];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      next_blk[0] = blk[i];
+      fetch(i, i < 2 ? first[i] : raw[i - 2]);
+    }
+    convert(0, first[0]);
+    convert(1, first[1]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  } else {
+    // (the blocks of all three tiles in one scalar round trip)
+    int blk[3][G::kPieces];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int u = 0; u < G::kPieces; ++u) blk[i][u] = table[piece_pos(i, u) >> lbs];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+#pragma unroll
+      for (int u = 0; u < G::kPieces; ++u) next_blk[u] = blk[i][u];
+      issue(i);
+    }
+    // q is consumed here so that no wait for it lands inside the loop
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks) asm volatile("" : "+v"(qb[ks]));
+    wait_vmem<2 * G::kPieces>();
+  }
+  constexpr std::integral_constant<int, 0> kFirst{};
+  constexpr std::integral_constant<int, kVF> kMid{};
+  constexpr std::integral_constant<int, kVF + kKF> kEnd{};
+  barrier();
+  if (wtiles > 0) products(kMid, kEnd, -1, [](auto) {});
+  if (wave >= 4) barrier();  // half a tile behind
+
+  // Y(t) and X(t); the scores of the tile after a wave's last one are not used.
+  // The loads' address arithmetic lies between X's products, a few instructions
+  // at a time; the scalar load of the blocks, which the compiler lets no LDS
+  // read be in flight beside, in Y.  X's issue priority: 2-6% at D = 128 FP16,
+  // -2 to -4% for INT8 and D = 64.
+  constexpr bool kPrio = D == 128 && !kInt8;
+  auto body = [&](int t, Raw& r) {
+    look_up(t + (kInt8 ? 4 : 3));
+    if constexpr (kInt8) convert(t + 2, r);
+    if (t < wtiles) softmax(t);
+    barrier();
+    if constexpr (kPrio) __builtin_amdgcn_s_setprio(1);
+    if (t < wtiles) {
+      products(kFirst, kEnd, t, [&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (kInt8) {
+          if constexpr (i == 2) fetch(t + 4, r);
+        } else if constexpr (i >= 1 && i % 3 == 1 && i / 3 < 2 * G::kPieces) {
+          issue_part(t + 3, i / 3);
+        }
+      });
+    } else if constexpr (kInt8) {
+      fetch(t + 4, r);
+    } else {
+      issue(t + 3);
+    }
+    if constexpr (kPrio) __builtin_amdgcn_s_setprio(0);
+    if constexpr (kInt8) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    else wait_vmem<2 * G::kPieces>();  // tile t + 2; t + 3 stays in flight
+    barrier();
+  };
+  int t = 0;
+  for (; t + 2 < ntiles; t += 2) {
+    body(t, raw[0]);
+    body(t + 1, raw[1]);
+  }
+  if (t + 1 < ntiles) body(t++, raw[0]);
+  // the last tile: no next one
+  if (t < wtiles) softmax(t);
+  barrier();
+  if (t < wtiles) products(kFirst, kMid, t, [](auto) {});
+  if (wave < 4) barrier();  // (the other group's last softmax)
+  if constexpr (!kInt8) wait_vmem<0>();  // no load may land after the workgroup has left its LDS
+
+  const float l = rows_sum<true>(l_run);  // the row's other half
+  if (!valid) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t* out = p.out + static_cast<size_t>(q0 + tok) * p.num_heads * D + head * D + 4 * half;
+#pragma unroll
+  for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const f16x4 r = {static_cast<_Float16>(o[dt][4 * b] * inv), static_cast<_Float16>(o[dt][4 * b + 1] * inv),
+                       static_cast<_Float16>(o[dt][4 * b + 2] * inv), static_cast<_Float16>(o[dt][4 * b + 3] * inv)};
+      *reinterpret_cast<f16x4*>(out + 32 * dt + 8 * b) = r;
+    }
+}
+
 // compute units of the current device (cached per device)
 int device_cus() {
   static int cus[64] = {0};
@@ -902,7 +1370,10 @@ int prefill(const rlk_attention_params* params, const rlk_prefill_attention_work
     return fail(RLK_EINVAL, "%s: null pointer argument", what);
   if (reinterpret_cast<uintptr_t>(p.q) % 16 != 0 || p.q_stride % 8 != 0)
     return fail(RLK_EINVAL, "%s: q rows must be 16-byte aligned (q_stride %d)", what, p.q_stride);
-  PrefillArgs a{p, w, scale16};
+  PrefillArgs a{};
+  a.p = p;
+  a.w = w;
+  a.scale16 = scale16;
   // the work's tiles are the reference's 32-row tiles (kPrefillTileQ); ours hold kBQ rows
   const int rows = w.max_q_tiles * RLK_PREFILL_TILE_Q;
   auto go = [&](auto kernel, auto shape) {
@@ -919,6 +1390,45 @@ int prefill(const rlk_attention_params* params, const rlk_prefill_attention_work
   // (INT8 with fp16 scales reads the dword that holds a scale and picks the
   // half by the key position's parity: even block sizes only)
   const bool dma_ok = dma_fits && (!int8 || !scale16 || p.kv.block_size % 2 == 0);
+  // The ping-pong kernel: a wave's loads stay in one cache block (a power of
+  // two of at least 8 rows); (token, head) rows and the cells of a block are
+  // counted in 32 bits (rows below 2^21: quot).  With fewer workgroups than
+  // half the compute units the kernel above is the faster one: its
+  // workgroups of 128 rows and one head are twice as many and start sooner (Llama
+  // heads, one prompt of 512 / 1024 / 2048 tokens, 64 / 128 / 256 workgroups:
+  // 20.6 / 33.0 / 60.3 against 17.3 / 30.3 / 99.6 us).
+  // RLK_TUNE_PREFILL_DMA = 2 forces this kernel, 1 the rule, 0 the register-staged one.
+  a.grp = p.num_heads / p.kv.num_kv_heads;
+  const int pp_tiles = static_cast<int>((static_cast<int64_t>(rows) * a.grp + 255) / 256);
+  const bool pp_ok = p.kv.block_size >= 8 && (p.kv.block_size & (p.kv.block_size - 1)) == 0 &&
+                     static_cast<int64_t>(rows) * a.grp < (int64_t{1} << 21) && pp_tiles <= 65535 &&
+                     static_cast<int64_t>(p.kv.num_kv_heads) * p.kv.block_size < (int64_t{1} << 30);
+  const int path = tune_knob(kPrefillDma, 1);
+  const bool pp_fills = !dma_ok || 2 * static_cast<int64_t>(pp_tiles) * p.kv.num_kv_heads * w.num_seqs > device_cus();
+  if (pp_ok && (path >= 2 || (path == 1 && pp_fills))) {
+    auto pp = [&](auto kernel, auto geo) -> int {
+      using G = decltype(geo);
+      const hipError_t e = grant_dynamic_lds(reinterpret_cast<const void*>(kernel), G::kLds);
+      if (e != hipSuccess)
+        return fail(RLK_EUNSUPPORTED, "%s: %d bytes of LDS refused (%s)", what, G::kLds, hipGetErrorString(e));
+      a.split = 1;  // kv heads x split: a multiple of the 8 XCDs
+      while (p.kv.num_kv_heads * a.split % 8 != 0) a.split *= 2;
+      a.inv_grp = 1.0f / static_cast<float>(a.grp);
+      a.inv_hkv = 1.0f / static_cast<float>(p.kv.num_kv_heads);
+      const dim3 grid(p.kv.num_kv_heads * a.split, (pp_tiles + a.split - 1) / a.split, w.num_seqs);
+      kernel<<<grid, G::kThreads, G::kLds, stream>>>(a);
+      return launch_status(what);
+    };
+    const PfKV kv = !int8 ? kPfFP16 : scale16 ? kPfInt8F16 : kPfInt8F32;
+    if (p.kv.head_dim == 64) {
+      if (kv == kPfFP16) return pp(prefill_pp_kernel<64, kPfFP16>, PfPP<64, false>{});
+      if (kv == kPfInt8F32) return pp(prefill_pp_kernel<64, kPfInt8F32>, PfPP<64, true>{});
+      return pp(prefill_pp_kernel<64, kPfInt8F16>, PfPP<64, true>{});
+    }
+    if (kv == kPfFP16) return pp(prefill_pp_kernel<128, kPfFP16>, PfPP<128, false>{});
+    if (kv == kPfInt8F32) return pp(prefill_pp_kernel<128, kPfInt8F32>, PfPP<128, true>{});
+    return pp(prefill_pp_kernel<128, kPfInt8F16>, PfPP<128, true>{});
+  }
   if (dma_ok && tune_knob(kPrefillDma, 1) != 0) {
     auto dma = [&](auto kernel, auto geo) -> int {
       using G = decltype(geo);

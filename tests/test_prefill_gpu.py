@@ -381,3 +381,63 @@ def test_prefill_attention_full_chip_repeats(torch_cuda, int8):
         s = (q[-n:, h * D:(h + 1) * D].float() @ k[:, h // (hq // hkv)].t().contiguous()) * D ** -0.5
         want = torch.softmax(s.masked_fill(mask, float("-inf")), -1) @ v[:, h // (hq // hkv)].contiguous()
         assert_close_f16(got[0][-n:, h * D:(h + 1) * D], want.cpu().numpy(), what=f"head {h}")
+
+
+@pytest.mark.parametrize("D,kv", [(64, "fp16"), (128, "fp16"), (64, "int8"), (128, "int8"),
+                                  (64, "int8_f16scale"), (128, "int8_f16scale")])
+@pytest.mark.parametrize("bs,hq,hkv", [(8, 7, 1), (16, 8, 8), (16, 28, 4), (32, 24, 3), (128, 16, 2)])
+def test_prefill_attention_ping_pong(torch_cuda, D, kv, bs, hq, hkv, kernel_path):
+    """The ping-pong kernel, forced at small grids: (token, head) rows that fill
+    workgroups only in part and straddle them, one tile of keys and many, tile
+    ends on and off 64 keys, blocks smaller and larger than a tile, kv heads that
+    do and do not divide the XCDs; against fp32 torch attention over the cache
+    (INT8: through fp16, as the kernel contract has it).  Written output rows only."""
+    if kernel_path != "dma":
+        pytest.skip("one kernel: the paths of this module do not apply")
+    torch = torch_cuda
+    from redline_amd import kernels as K
+    from redline_amd._lib import tune_knob
+    say(f"prefill ping-pong D={D} kv={kv} bs={bs} hq={hq} hkv={hkv}")
+    segs = [(0, 2), (63, 2), (0, 64), (64, 65), (200, 300), (0, 33), (447, 65), (5, 130)]
+    rng = np.random.default_rng(D + bs + hq)
+    g = torch.Generator(device="cuda").manual_seed(D + bs + hq)
+    need = [(s + n + bs - 1) // bs for s, n in segs]
+    S, T, G = len(segs), sum(n for _, n in segs), hq // hkv
+    cache = K.KVCache(1, sum(need) + 1, hkv, D, bs, K.KVDType.kFP16 if kv == "fp16" else K.KVDType.kINT8,
+                      scale_dtype=K.SCALE_F16 if kv == "int8_f16scale" else K.SCALE_F32)
+    for i, t in enumerate(x for x in cache.tensors(0) if x is not None):
+        if t.dtype == torch.int8:
+            t.copy_(torch.randint(-127, 128, t.shape, generator=g, device="cuda", dtype=torch.int8))
+        elif i < 2:
+            t.normal_(generator=g)
+        else:
+            t.uniform_(0.008, 0.018, generator=g)
+    pool = rng.permutation(np.arange(1, sum(need) + 1, dtype=np.int32))
+    bb = ra.BatchBuilder(T, S, S, max(need), bs, 1)
+    tables, at = [], 0
+    for (s, n), k in zip(segs, need):
+        tables.append(pool[at:at + k])
+        bb.add(np.zeros(n, np.int32), s, n, None, pool[at:at + k])
+        at += k
+    meta, shape, lay = bb.write()
+    d_meta = dev(torch, meta)
+    stride = (hq + 2 * hkv) * D
+    q = (1.5 * torch.randn((T, stride), generator=g, device="cuda")).half()
+    with tune_knob("RLK_TUNE_PREFILL_DMA", 2):
+        got = run_prefill(torch, K, q, stride, hq, D ** -0.5, cache.layer(0), d_meta[lay["block_tables"]:],
+                          max(need), d_meta[lay["positions"]:], d_meta, lay, shape, T, D,
+                          scale16=kv == "int8_f16scale")
+    k, v, ks, vs = cache.tensors(0)
+    at = 0
+    for (s, n), t in zip(segs, tables):
+        idx = torch.from_numpy(t.astype(np.int64)).cuda()
+        rows = lambda x, sc: (x[idx].float() if sc is None else  # noqa: E731
+                              (x[idx].float() * sc[idx].float()[..., None]).half().float()
+                              ).transpose(1, 2).reshape(-1, hkv, D)[:s + n]
+        kk, vv = rows(k, ks), rows(v, vs)
+        mask = torch.arange(s + n, device="cuda")[None] > s + torch.arange(n, device="cuda")[:, None]
+        for h in range(hq):
+            sc = (q[at:at + n, h * D:(h + 1) * D].float() @ kk[:, h // G].t().contiguous()) * D ** -0.5
+            want = torch.softmax(sc.masked_fill(mask, float("-inf")), -1) @ vv[:, h // G].contiguous()
+            assert_close_f16(got[at:at + n, h * D:(h + 1) * D], want.cpu().numpy(), what=f"segment {s}+{n} head {h}")
+        at += n
