@@ -1014,7 +1014,7 @@ __global__ __launch_bounds__(kThreads, (G <= 4 ? 4 : 2)) void decode_attention_k
                       min((ctx + kPart - 1) / kPart, w.max_partitions), part, kvh);
 }
 
-// Merges the split-K partials of one (item, head), one lane per output dim
+// Merges the split-K partials of one (item, head), one lane per output dim (and group of rows)
 // (the merge rule of attention.cu:193-210).  A partition's partial row is
 // sum_k e^(s_k - m_i) v_k, not divided by its sum l_i; the output is
 // sum_i e^(m_i - M) row_i / sum_i e^(m_i - M) l_i with M = max_i m_i.  The
@@ -1027,60 +1027,68 @@ __global__ __launch_bounds__(kThreads, (G <= 4 ? 4 : 2)) void decode_attention_k
 // round trips.  Entries past the count are never used (they may hold anything).
 constexpr int kReduceMaxParts = 4096;  // weights kept in LDS (contexts up to 1M keys)
 
-template <int D, bool kRuns>
-__global__ __launch_bounds__(D) void decode_reduce_kernel(AttnArgs args) {
+template <int D, bool kRuns, int kGroups>
+__global__ __launch_bounds__((D * kGroups)) void decode_reduce_kernel(AttnArgs args) {
   // kRuns: slots absorbed by a persistent workgroup's run hold the sum -1
   // and take no part (weight marker -1, rows never accumulated); slot 0 is
   // always a run's own, so only it is requested before the slots' states
-  // are known, and later rows past the count or of absorbed slots re-read it
+  // are known, and later rows past the count or of absorbed slots re-read it.
+  // Thread (g, d) takes dim d of rows g, g + kGroups, ...
   constexpr int kEarly = kRuns ? 1 : 4, kLate = kRuns ? 31 : 28;
-  constexpr int kUnroll = 8;
+  constexpr int kUnroll = 8, kThr = D * kGroups, kWv = kThr / kWave;
   const rlk_attention_params& p = args.p;
   const rlk_decode_attention_work& w = args.w;
   __shared__ float wgt[kReduceMaxParts];
-  __shared__ float part_red[D / kWave];
-  const int item = blockIdx.x, h = blockIdx.y, d = threadIdx.x, lane = d % kWave, wv = d / kWave;
+  __shared__ float part_red[kWv];
+  __shared__ float acc[kGroups > 1 ? kGroups - 1 : 1][D];
+  const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid % kWave, wv = tid / kWave;
+  const int g = kGroups > 1 ? tid / D : 0, d = tid % D;
   const int mp = w.max_partitions;
   const int64_t base = (static_cast<int64_t>(item) * p.num_heads + h) * mp;
   const float* src = w.ws_out + base * D + d;
-  const float m0 = d < mp ? w.ws_max[base + d] : -FLT_MAX;
-  const float l0 = d < mp ? w.ws_sum[base + d] : 0.f;
+  const float m0 = tid < mp ? w.ws_max[base + tid] : -FLT_MAX;
+  const float l0 = tid < mp ? w.ws_sum[base + tid] : 0.f;
   // every wave's view of slots 0..63 (wave 0's own l0)
   const float lw = kRuns && wv > 0 && lane < mp ? w.ws_sum[base + lane] : l0;
+  auto slot = [&](int u) { return g + kGroups * u; };  // this thread's u-th row
   float v0[kEarly];
 #pragma unroll
-  for (int u = 0; u < kEarly; ++u) v0[u] = u < mp ? src[static_cast<int64_t>(u) * D] : 0.f;
+  for (int u = 0; u < kEarly; ++u)
+    v0[u] = slot(u) < mp ? src[static_cast<int64_t>(kRuns ? 0 : slot(u)) * D] : 0.f;
   const int token = w.item_token[item];
   const int ctx = p.positions[token] + 1;
   const int num_parts = min((ctx + kPart - 1) / kPart, mp);
   if (num_parts <= 1) return;  // uniform: written directly by the attention kernel
   // bit j: slot j < 64 holds a partial of its own
   const uint64_t own = kRuns ? __ballot(lane < num_parts && !(lw < 0.f)) : ~0ull;
+  auto row = [&](int j) {
+    j = min(j, num_parts - 1);
+    return src[static_cast<int64_t>(kRuns && j < 64 && !((own >> j) & 1) ? 0 : j) * D];
+  };
+  // (kRuns: groups past the first have no early row of their own)
+  constexpr int kFirst = kRuns && kGroups > 1 ? 0 : kEarly;
   float v1[kLate];
 #pragma unroll
-  for (int u = 0; u < kLate; ++u) {
-    const int j = min(kEarly + u, num_parts - 1);
-    v1[u] = src[static_cast<int64_t>(kRuns && j < 64 && !((own >> j) & 1) ? 0 : j) * D];
-  }
+  for (int u = 0; u < kLate; ++u) v1[u] = row(slot(kFirst + u));
 
-  float mx = d < num_parts && !(kRuns && l0 < 0.f) ? m0 : -FLT_MAX;
-  for (int i = d + D; i < num_parts; i += D)
+  float mx = tid < num_parts && !(kRuns && l0 < 0.f) ? m0 : -FLT_MAX;
+  for (int i = tid + kThr; i < num_parts; i += kThr)
     if (!(kRuns && w.ws_sum[base + i] < 0.f)) mx = fmaxf(mx, w.ws_max[base + i]);
   mx = rows_max<true>(rows_max<false>(group_max<16>(mx)));
   if (lane == 0) part_red[wv] = mx;
   __syncthreads();
   mx = part_red[0];
 #pragma unroll
-  for (int i = 1; i < D / kWave; ++i) mx = fmaxf(mx, part_red[i]);
+  for (int i = 1; i < kWv; ++i) mx = fmaxf(mx, part_red[i]);
   __syncthreads();  // part_red is reused below
   float total = 0.f;
-  if (d < num_parts) {
+  if (tid < num_parts) {
     const float f = __expf(m0 - mx);
     const bool absorbed = kRuns && l0 < 0.f;
-    wgt[d] = absorbed ? -1.f : f;
+    wgt[tid] = absorbed ? -1.f : f;
     if (!absorbed) total = f * l0;
   }
-  for (int i = d + D; i < num_parts; i += D) {
+  for (int i = tid + kThr; i < num_parts; i += kThr) {
     const float li = w.ws_sum[base + i];
     const float f = __expf(w.ws_max[base + i] - mx);
     const bool absorbed = kRuns && li < 0.f;
@@ -1092,26 +1100,30 @@ __global__ __launch_bounds__(D) void decode_reduce_kernel(AttnArgs args) {
   __syncthreads();
   total = part_red[0];
 #pragma unroll
-  for (int i = 1; i < D / kWave; ++i) total += part_red[i];
+  for (int i = 1; i < kWv; ++i) total += part_red[i];
 
   float o = 0.f;
+  auto add = [&](int j, float v) {
+    if (j < num_parts && !(kRuns && wgt[j] == -1.f)) o += wgt[j] * v;
+  };
 #pragma unroll
-  for (int u = 0; u < kEarly; ++u)
-    if (u < num_parts && !(kRuns && wgt[u] == -1.f)) o += wgt[u] * v0[u];
+  for (int u = 0; u < kFirst; ++u) add(slot(u), v0[u]);
 #pragma unroll
-  for (int u = 0; u < kLate; ++u)
-    if (kEarly + u < num_parts && !(kRuns && wgt[kEarly + u] == -1.f)) o += wgt[kEarly + u] * v1[u];
-  int i = kEarly + kLate;
-  for (; i + kUnroll <= num_parts; i += kUnroll) {
+  for (int u = 0; u < kLate; ++u) add(slot(kFirst + u), v1[u]);
+  for (int i = kFirst + kLate; slot(i) < num_parts; i += kUnroll) {
     float v[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) v[u] = src[static_cast<int64_t>(i + u) * D];
+    for (int u = 0; u < kUnroll; ++u) v[u] = row(slot(i + u));
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
-      if (!(kRuns && wgt[i + u] == -1.f)) o += wgt[i + u] * v[u];
+    for (int u = 0; u < kUnroll; ++u) add(slot(i + u), v[u]);
   }
-  for (; i < num_parts; ++i)
-    if (!(kRuns && wgt[i] == -1.f)) o += wgt[i] * src[static_cast<int64_t>(i) * D];
+  if constexpr (kGroups > 1) {
+    if (g > 0) acc[g - 1][d] = o;
+    __syncthreads();
+    if (g > 0) return;
+#pragma unroll
+    for (int i = 0; i < kGroups - 1; ++i) o += acc[i][d];
+  }
   reinterpret_cast<_Float16*>(p.out)[static_cast<int64_t>(token) * p.num_heads * D + h * D + d] =
       static_cast<_Float16>(o / total);
 }
@@ -1166,11 +1178,17 @@ bool launch_d(const AttnArgs& a, int G, bool int8, hipStream_t stream) {
     default: return false;
   }
   if (a.w.max_partitions > 1) {
+    // One thread group requests 32 rows in two batches, and 8 a round trip after
+    // that: past 32 partitions four groups share them (4 items x 28 heads of up to
+    // 128 partitions: the call 31.6 -> 29.9 us, one 32768-key item x 32 heads 35.5 -> 33.3).
     const dim3 grid(a.w.num_items, a.p.num_heads);
+    const bool wide = a.w.max_partitions > 32;
     if (runs) {
-      decode_reduce_kernel<D, true><<<grid, D, 0, stream>>>(a);
+      if (wide) decode_reduce_kernel<D, true, 4><<<grid, 4 * D, 0, stream>>>(a);
+      else decode_reduce_kernel<D, true, 1><<<grid, D, 0, stream>>>(a);
     } else {
-      decode_reduce_kernel<D, false><<<grid, D, 0, stream>>>(a);
+      if (wide) decode_reduce_kernel<D, false, 4><<<grid, 4 * D, 0, stream>>>(a);
+      else decode_reduce_kernel<D, false, 1><<<grid, D, 0, stream>>>(a);
     }
   }
   return true;
