@@ -1128,15 +1128,24 @@ __global__ __launch_bounds__((D * kGroups)) void decode_reduce_kernel(AttnArgs a
       static_cast<_Float16>(o / total);
 }
 
-// The persistent form (two workgroups per CU) serves batches of up to
-// kMaxItemsLds decode items, the grid form larger ones.  RLK_TUNE_ATTN_PERSIST
-// overrides: workgroups per CU for the persistent form, or 0 for the grid form.
+// The persistent form (two workgroups per CU) pays for its pipeline with a
+// longer start (the items' prefix sums, two units' table entries): it serves
+// calls of many units ((item, kv head, partition) triples of the grid) and up to
+// kMaxItemsLds decode items, the grid form the others.  Measured (us, grid
+// against persistent): one 1300-key item, 8 kv heads of 128 8.8 / 11.6 (FP16),
+// 8.0 / 9.4 (INT8); 32 items to 1024 keys, 1024 units, 21.0 / 26.0, 16.2 / 19.6;
+// 2048 units (4 items to 32768 keys, 4 kv heads) 44.7 / 44.8, 27.2 / 29.9; 4096
+// units 83.2 / 79.1 and 71 / 52 (32 items to 8192 keys).  INT8 at D = 64 crosses
+// below 2048 units (15.6 / 17.2 at 1024, 22.0 / 20.1 at 2048).
+// RLK_TUNE_ATTN_PERSIST overrides: workgroups per CU for the persistent form, or
+// 0 for the grid form.
 // Returns whether the partials were written by runs (absorbed slots marked).
 template <int D, int G, bool kMma>
 bool launch_gm(const AttnArgs& a, bool int8, hipStream_t stream) {
-  const int mode = tune_knob(kAttnPersist, 2);
+  const int64_t units = static_cast<int64_t>(a.w.num_items) * a.w.max_partitions * a.p.kv.num_kv_heads;
+  const int64_t few = static_cast<int64_t>(compute_units()) * (D == 64 && int8 ? 4 : 8);
+  const int mode = tune_knob(kAttnPersist, units <= few ? 0 : 2);
   if (mode > 0 && a.w.num_items <= kMaxItemsLds) {
-    const int64_t units = static_cast<int64_t>(a.w.num_items) * a.w.max_partitions * a.p.kv.num_kv_heads;
     const int blocks = static_cast<int>(std::min<int64_t>(units, static_cast<int64_t>(compute_units()) * mode));
     if (int8) {
       decode_attention_persistent<D, G, true, kMma><<<blocks, kThreads, 0, stream>>>(a);
