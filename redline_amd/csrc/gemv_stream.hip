@@ -46,7 +46,7 @@ struct StreamArgs {
   int gsh;           // kInt4Small: log2(group_size / 32)
   int rows_wg;       // weight rows of a workgroup (at most 16)
   int so_bytes;      // LDS bytes of the staged scales (whole KiB); as many for the offsets
-  int so_dma;        // the workgroup's scales and offsets are 16-byte aligned
+  int so_dma;        // the workgroup's scales and offsets are 16-byte aligned, the arrays whole dwords
   int so_shift, so_mask;  // piece p of row r is staged at p ^ ((r >> so_shift) & so_mask)
   float inv_pieces;  // 1 / 16-byte pieces of a row (1 where nothing is swizzled)
 };
@@ -441,7 +441,10 @@ int launch_gemv_stream(const StreamCall& c, hipStream_t stream) {
     return launch_rows<kInt8>(s, stream);
   }
   a.groups = c.k / c.group_size;
-  s.so_dma = (reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.offsets)) % 16 == 0;
+  // (the buffers' bounds are checked by dwords: an odd number of scales, as
+  // odd n and odd groups give, would have the last one half outside)
+  s.so_dma = (reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.offsets)) % 16 == 0 &&
+             static_cast<int64_t>(a.n) * a.groups % 2 == 0;
   s.nsteps = (s.nchunks + 1) / 2;
   if (c.group_size % 128 == 0) {
     const int gq = c.group_size / 128;

@@ -271,3 +271,25 @@ def test_gemv_w4_stream_shapes(torch_cuda, n, k, g, m):
     assert_close_f16(got16, want.astype(np.float16), what="stream fp16")
     if gated is not None:
         assert_close_f16(gated, oracle.gemv_w4a16_swiglu(x, packed, s, o, g), what="stream swiglu")
+
+
+@pytest.mark.parametrize("n,k,g", [(2047, 384, 128), (4095, 1152, 128), (4095, 128, 128)])
+@pytest.mark.parametrize("m", [1, 17])
+def test_gemv_w4_stream_odd_scales(torch_cuda, n, k, g, m):
+    """The streaming kernel where the number of scales is odd and a workgroup's
+    first scale lies on 16 bytes (8 or 16 rows per workgroup at 256 compute
+    units; arrays 16-byte aligned): the last row's last scale and offset are
+    the first half of a dword.  The default policy; every column, and the last
+    one by itself (x of ones there, so that its product is the row's sum).
+    Tolerance as test_gemv_w4_stream_shapes."""
+    torch = torch_cuda
+    say(f"gemv_w4 stream odd scales n={n} k={k} g={g} m={m}")
+    rng = np.random.default_rng(n + k + m)
+    packed, s, o, _ = int4_linear(rng, n, k, g, dense=False)
+    s[-1, -1], o[-1, -1] = 0.5, -3.0  # a lost scale or offset changes the last column at once
+    x = randn_f16(rng, (m, k))
+    x[0] = 1.0
+    want = oracle.gemv_w4a16(x, packed, s, o, g)
+    got = run_gemv(torch, x, packed, s, o, g, f32=True)
+    assert rel_max_err(got[:, -1], want[:, -1]) <= 1e-5
+    assert rel_max_err(got, want) <= 1e-5
