@@ -851,7 +851,10 @@ __global__ __launch_bounds__((64 * kslice_max_waves<CPW, MT>())) void gemv_w4_ks
 // per 8 codes, int8x8_to_f16_biased); each tile's sum starts from -1152
 // sum(x) of the slice, so the products leave x . code.  The row scale and
 // the bias apply once, to the reduced sum (gemv_weight_only.cu:36).
-template <int CPW, int U, int MT, int MODE>
+// kTail: n may end inside a tile, and the codes are exact (4 VALU more per 8
+// codes): the bias costs fp32 sum bits (2.5e-6 of the result at K = 4096 against
+// 4e-7), which products of such n, the pair kernel's otherwise, do not give up.
+template <int CPW, int U, int MT, int MODE, bool kTail>
 __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a) {
   constexpr int P = CPW * U;  // ring depth in lines: U tiles
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -861,7 +864,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
   const int r16 = lane & 15, qd = lane >> 4;
   const bool low = (lane & 8) == 0;
   const int T = a.cpp;  // tiles per workgroup, a multiple of U
-  const int ntiles = (a.n + 15) / 16;
+  const int ntiles = kTail ? (a.n + 15) / 16 : a.n / 16;
   const int tile0 = blockIdx.x * T;
   f32x4* red = reinterpret_cast<f32x4*>(lds);  // [T][nw][MT][64 lanes]
   const int kb = a.k;
@@ -878,9 +881,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
     const int t = tile0 + q / CPW;
     const __amdgpu_buffer_rsrc_t res = (q < nq && t < ntiles) ? wres : none;
     const int soff = t * 16 * kb + (l0 + q % CPW) * 128;
-    const int last = (a.n - 1 - t * 16) * kb;  // rows past n re-read the last one
-    ring[s][0] = __builtin_amdgcn_raw_buffer_load_b128(res, min(vo0, last) + pc0, soff, kNtLoad);
-    ring[s][1] = __builtin_amdgcn_raw_buffer_load_b128(res, min(vo1, last) + pc1, soff, kNtLoad);
+    const int last = (kTail ? min(a.n - 1 - t * 16, 15) : 15) * kb;  // rows past n re-read the last one
+    ring[s][0] = __builtin_amdgcn_raw_buffer_load_b128(res, (kTail ? min(vo0, last) : vo0) + pc0, soff, kNtLoad);
+    ring[s][1] = __builtin_amdgcn_raw_buffer_load_b128(res, (kTail ? min(vo1, last) : vo1) + pc1, soff, kNtLoad);
   };
 
   // x of the slice in the A layout above, staged as in the INT4 kernel
@@ -912,17 +915,18 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
   }
 #pragma unroll
   for (int p = 0; p < P; ++p) fetch(p, p);
-  // -1152 sum(x) of the slice per activation row (all 16 columns equal)
+  // -1152 sum(x) of the slice per activation row (all 16 columns equal); 0 for exact codes
   const f16x8 kM1152 = {-1152, -1152, -1152, -1152, -1152, -1152, -1152, -1152};
   f32x4 base[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     base[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (!kTail)
 #pragma unroll
-    for (int c = 0; c < CPW; ++c)
+      for (int c = 0; c < CPW; ++c)
 #pragma unroll
-      for (int st = 0; st < 4; ++st)
-        base[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[c][mt][st], kM1152, base[mt], 0, 0, 0);
+        for (int st = 0; st < 4; ++st)
+          base[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[c][mt][st], kM1152, base[mt], 0, 0, 0);
   }
   __syncthreads();  // every wave is done with its staging rows (they hold partial sums next)
 
@@ -948,7 +952,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
           const u32x4 w = words[st >> 1];
-          const f16x8 q = int8x8_to_f16_biased((st & 1) ? u32x2{w.z, w.w} : u32x2{w.x, w.y});
+          const u32x2 codes = (st & 1) ? u32x2{w.z, w.w} : u32x2{w.x, w.y};
+          const f16x8 q = kTail ? int8x8_to_f16(codes) : int8x8_to_f16_biased(codes);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
             acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[c][mt][st], q, acc[mt], 0, 0, 0);
@@ -962,7 +967,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
   for (int t = wave; t < T; t += nw) {
     const int row = (tile0 + t) * 16 + r16;
     if (tile0 + t >= ntiles) break;
-    const float sc = static_cast<float>(__builtin_bit_cast(_Float16, a.scales[min(row, a.n - 1)]));
+    const float sc = static_cast<float>(__builtin_bit_cast(_Float16, a.scales[kTail ? min(row, a.n - 1) : row]));
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       f32x4 sum = red[((t * nw) * MT + mt) * kWave + lane];
@@ -1258,7 +1263,8 @@ int launch_kslice_w8(W4Args a, hipStream_t stream) {
   if (lds_for(T) > kLdsBudget) return kNoFit;
   a.cpp = T;
   const size_t lds = lds_for(T);
-  auto kernel = gemv_w8_kslice_kernel<CPW, U, MT, MODE>;
+  auto kernel = a.n % 16 == 0 ? gemv_w8_kslice_kernel<CPW, U, MT, MODE, false>
+                              : gemv_w8_kslice_kernel<CPW, U, MT, MODE, true>;
   if (lds > 64 * 1024) {
     const hipError_t e = grant_dynamic_lds(reinterpret_cast<const void*>(kernel), kLdsBudget);
     if (e != hipSuccess)

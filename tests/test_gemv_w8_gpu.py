@@ -174,3 +174,22 @@ def test_gemv_w8_stream_and_row_tails(torch_cuda, cfg, n, k, m):
         got16 = run_w8(torch_cuda, x, q, s, bias, False)
     assert rel_max_err(got, want) <= 1e-4
     assert_close_f16(got16, want, what="w8 stream f16")
+
+
+@pytest.mark.parametrize("n,k", [(97, 4096), (4097, 4096), (10007, 2048)])
+@pytest.mark.parametrize("m", [1, 17])
+def test_gemv_w8_row_tails_fp32_error(torch_cuda, n, k, m):
+    """The default policy where n ends inside a 16-row tile: the codes enter the
+    products exactly.  A biased code (1152 + code) makes each partial sum about
+    16 times the result's size, and its fp32 rounding with it (2.5e-6 of the
+    result).  Exact codes: 16 MFMA and up to 8 slice sums, each rounded at 2^-24
+    of a partial sum no larger than the result, about 6e-8 x sqrt(24) = 3e-7;
+    three times that."""
+    say(f"gemv_w8 row tails fp32 n={n} k={k} m={m}")
+    rng = np.random.default_rng(n + k + m)
+    q = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    s = rng.uniform(0.001, 0.01, n).astype(np.float16)
+    x = randn_f16(rng, (m, k))
+    want = (x.astype(np.float64) @ q.T.astype(np.float64)) * s.astype(np.float64)
+    got = run_w8(torch_cuda, x, q, s, None, True).astype(np.float64)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
