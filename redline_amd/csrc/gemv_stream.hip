@@ -409,7 +409,10 @@ int launch_rows(const StreamArgs& s, hipStream_t stream) {
   constexpr bool k8 = KIND == kInt8;
   if constexpr (!k8)
     if (m <= 2) return launch<KIND, 2, 4>(s, stream);
-  if (m <= 4) return launch<KIND, 4, 4>(s, stream);
+  // Groups of 32 and 64 at one step per wave: 4 steps in flight are 3 too many
+  // (groups of 32, m = 4, k = 2048, slab / streaming time at n = 28672 and 65536:
+  // 0.97 and 0.94 with 4 rows staged and 4 steps in flight).
+  if (m <= 4 && !(KIND == kInt4Small && s.nsteps <= kMaxWaves)) return launch<KIND, 4, 4>(s, stream);
   if (m <= 8) return launch<KIND, 8, k8 ? 4 : 2>(s, stream);
   if (m <= 16) return launch<KIND, 16, 2>(s, stream);
   return launch<KIND, 32, k8 ? 2 : 1>(s, stream);

@@ -857,6 +857,9 @@ __global__ __launch_bounds__((64 * kslice_max_waves<CPW, MT>())) void gemv_w4_ks
 template <int CPW, int U, int MT, int MODE, bool kTail>
 __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a) {
   constexpr int P = CPW * U;  // ring depth in lines: U tiles
+  // (clamped row offsets are part of the schedule with two activation tiles: 28672 x
+  // 4096, m = 32: 25.1 us with, 26.1 without; with one tile 65536 x 1024: 17.9 / 17.4)
+  constexpr bool kClamp = kTail || MT == 2;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int threads = blockDim.x, nw = threads / 64;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -881,9 +884,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
     const int t = tile0 + q / CPW;
     const __amdgpu_buffer_rsrc_t res = (q < nq && t < ntiles) ? wres : none;
     const int soff = t * 16 * kb + (l0 + q % CPW) * 128;
-    const int last = (kTail ? min(a.n - 1 - t * 16, 15) : 15) * kb;  // rows past n re-read the last one
-    ring[s][0] = __builtin_amdgcn_raw_buffer_load_b128(res, (kTail ? min(vo0, last) : vo0) + pc0, soff, kNtLoad);
-    ring[s][1] = __builtin_amdgcn_raw_buffer_load_b128(res, (kTail ? min(vo1, last) : vo1) + pc1, soff, kNtLoad);
+    [[maybe_unused]] const int last = (a.n - 1 - t * 16) * kb;  // rows past n re-read the last one
+    ring[s][0] = __builtin_amdgcn_raw_buffer_load_b128(res, (kClamp ? min(vo0, last) : vo0) + pc0, soff, kNtLoad);
+    ring[s][1] = __builtin_amdgcn_raw_buffer_load_b128(res, (kClamp ? min(vo1, last) : vo1) + pc1, soff, kNtLoad);
   };
 
   // x of the slice in the A layout above, staged as in the INT4 kernel
@@ -1128,15 +1131,48 @@ int launch_stream(const W4Args& a, hipStream_t s) {
       StreamCall{a.x, a.w, a.scales, a.offsets, a.bias, a.y, a.m, a.n, a.k, a.group_size, MODE, a.y_ld}, s);
 }
 
+// Groups of 32 and 64 need a scale per MFMA step: the streaming kernel's
+// transposed codes against the slab kernel's 4-byte loads (k = 4096, groups of
+// 32, m = 1 / 8 / 32: n = 4096 6.4 / 7.1 / 9.6 against 17.4 / 21.6 / 40.5 us;
+// n = 28672 26.7 / 29.1 / 55 against 41 / 42 / 48, equal at m = 16).  Above m = 8
+// every tile's x counts: up to two tiles per compute unit at any K, up to four
+// where K is long enough to pay for the starts or short enough that the slab
+// kernel's is dearer (slab / streaming time, groups of 64, m = 16 / 32; n = 12288:
+// k = 896 1.03 / 1.08, 1152 0.74 / 0.86, 2560 0.93 / 0.89, 3072 0.96 / 0.95, 3584 0.98 /
+// 1.01, 4096 1.06 / 1.14; n = 16384: 512 1.09 / 1.08, 640 0.96 / 0.94, 2048 0.67 / 0.70,
+// 3584 0.92 / 0.85, 3840 1.03 / 0.93, 4352 1.06 / 0.91, 6144 1.21 / 1.05).
+bool stream_small_groups(int m, int k, int tiles, int cus) {
+  if (m <= 8 || tiles <= 2 * cus) return true;
+  if (tiles <= 3 * cus) return k < 1024 || k >= (m <= 16 ? 3072 : 3584);
+  return tiles <= 4 * cus && (k <= 512 || k >= (m <= 16 ? 3584 : 5376));
+}
+
+// Between one and two tiles per compute unit the streaming kernel re-reads x
+// and starts twice: it beats the pair kernel (an even number of chunks) or the
+// slab kernel (an odd one) where K is long.  n = 8192, theirs / streaming time:
+//   m = 1 / 4 / 6: k = 2048 0.84 / 0.79 / 0.97, 2560 0.99 / 1.00 / 1.13, 3072 0.94 /
+//   0.95 / 1.17, 3584 1.11 / 1.12 / 1.33, 4096 1.08 / 1.10 / 1.34;
+//   m = 8, the pair kernel's last row count with 4 pairs in flight: 1.02-1.44 at
+//   any k;
+//   m = 9 / 16 / 17 / 32, even: k = 256 0.95 / 0.95 / 0.94 / 0.97, 768 0.95 / 1.13 /
+//   1.22 / 1.34, 1280 0.88 / 0.94 / 1.04 / 1.21, 2304 0.99 / 1.08 / 1.05 / 1.33, 3328
+//   1.23 / 1.33 / 1.28 / 1.65; odd: 640 0.96 / 1.06 / 1.10 / 1.14, 1152 0.79 / 0.82 /
+//   0.94 / 1.00, 2176 0.79 / 0.80 / 0.87 / 0.98, 3200 0.90 / 0.93 / 1.00 / 1.14, 3712
+//   0.99 / 0.99 / 1.06 / 1.21.
+// At three tiles the two are equal at k = 5120, and beyond that re-reading x per
+// tile costs the streaming kernel more (n = 28672, k = 4096, m = 1: 19 against 14.3 us).
+bool stream_two_tiles(int m, int k) {
+  if (m <= 8) return m == 8 || k > (m > 4 ? 2048 : 3200);
+  const bool pairs = k % 256 == 0;
+  if (m <= 16) return k > (pairs ? 2048 : 3200);
+  return pairs ? k > 512 : k < 1024 || k >= 3200;
+}
+
 template <int KC, int MT, int MODE>
 int launch_cfg(const W4Args& a, int cfg, hipStream_t s) {
   int st = kNoFit;
   const int tiles = (a.n + 15) / 16, cus = compute_units();
-  // Groups of 32 and 64 need a scale per MFMA step: the streaming kernel's
-  // transposed codes against the slab kernel's 4-byte loads (k = 4096, groups of
-  // 32, m = 1 / 8 / 32: n = 4096 6.4 / 7.1 / 9.6 against 17.4 / 21.6 / 40.5 us;
-  // n = 28672 26.7 / 29.1 / 55 against 41 / 42 / 48, equal at m = 16).
-  if (cfg == 16 || (KC == 32 && cfg == 0 && (a.m <= 8 || tiles <= 4 * cus))) st = launch_stream<MODE>(a, s);
+  if (cfg == 16 || (KC == 32 && cfg == 0 && stream_small_groups(a.m, a.k, tiles, cus))) st = launch_stream<MODE>(a, s);
   if (st != kNoFit) return st;
   if constexpr (KC == 128) {
     switch (cfg) {
@@ -1160,20 +1196,19 @@ int launch_cfg(const W4Args& a, int cfg, hipStream_t s) {
         // loads of a compute unit in flight where the pair kernel has one wave
         // (k = 4096, n = 4096, m = 1 / 4: 5.5 / 6.1 against 8.4 / 11.4 us) and
         // whose wait for x is shorter than the K-slice kernel's (m = 8 / 16 /
-        // 32: 5.9 / 7.1 / 8.8 against 7.8 / 7.8 / 10.3).  Up to two tiles per
-        // compute unit it also beats the pair kernel (n = 8192, k = 5120: 9.6
-        // against 10.9 at m = 1, 20.3 against 36.6 at m = 32); at three they
-        // are equal and beyond that re-reading x per tile costs it more (n =
-        // 28672, k = 4096, m = 1: 19 against 14.3).
+        // 32: 5.9 / 7.1 / 8.8 against 7.8 / 7.8 / 10.3), but for a slice of one
+        // or two of its steps at m = 9 .. 16 (n = 4096, m = 16, k = 1024 / 1536 /
+        // 2048 / 2560: the K-slice kernel at 1.05 / 0.96 / 0.87 / 0.97 of its time).
         // Many rows, measured at the Llama-3.1-8B gate_up shape: the pair
         // kernel with 4 pairs in flight below m = 8 (m = 4: 14.5-14.8 against
         // 15.1-15.9 us); the K-slice kernel with two tiles' pairs in flight from
         // m = 8 on, where staging x per workgroup and reading it back from LDS
         // per chunk cost the most (m = 8: 15.2-15.3 against 15.4-15.6 us, m =
-        // 16: 15.5-15.7 against 17.3-17.5, m = 32: 20.2 against 25.7)
-        if (tiles <= cus) st = launch_stream<MODE>(a, s);
+        // 16: 15.5-15.7 against 17.3-17.5, m = 32: 20.2 against 25.7).
+        if (a.m > 8 && a.m <= 16 && a.k > 1024 && a.k <= 2048) st = launch_kslice<4, 2, MT, MODE>(a, s);
+        if (st == kNoFit && tiles <= cus) st = launch_stream<MODE>(a, s);
         if (st == kNoFit && a.m >= 8) st = launch_kslice<4, 2, MT, MODE>(a, s);
-        if (st == kNoFit && tiles <= 2 * cus) st = launch_stream<MODE>(a, s);
+        if (st == kNoFit && tiles <= 2 * cus && stream_two_tiles(a.m, a.k)) st = launch_stream<MODE>(a, s);
         if (st == kNoFit)
           st = a.m <= 8 ? launch_pairs<4, MT, MODE>(a, s) : launch_pairs<2, MT, MODE>(a, s);
         break;
@@ -1279,14 +1314,23 @@ int launch_kslice_w8(W4Args a, hipStream_t stream) {
 // one tile's lines in flight where it fits (K a multiple of 512 up to 4096: at
 // the Llama-3.1-8B gate_up shape 23.2 / 23.4 / 23.6 / 26.4 us at m = 1 / 8 /
 // 16 / 32 against 25.0 / 25.7 / 26.5 / 30.7 for the pair kernel, same run).
-// Other K: the streaming kernel up to two tiles per compute unit (n = k = 5120,
-// m = 1 / 8 / 32: 10.4 / 13.0 / 22.9 against 12.7 / 14.9 / 28.2 us; n = 3584,
-// k = 18944: 14-15 / 18-20 / 33 against 38.7 / 59 / 134; at n = 10240 16.2 /
-// 20.4 / 35 against 16.2 / 18.0 / 28.3), else the pair kernel's INT8 form with
-// P = 4 pairs in flight (equal to or faster than 2 and 8).  RLK_TUNE_W8_CFG =
-// 1, 2, 3 selects the pair kernel with P = 2, 4, 8, 4, 5, 6 the K-slice kernel
-// with (lines per slice, tiles in flight) = (4, 1), (4, 2), (2, 2), and 7 the
-// streaming kernel.
+// Where n ends inside a tile the other choice is the pair kernel, which a
+// workgroup of k / 512 waves only beats if it has enough of them for its tiles
+// (pair / K-slice time, m = 1 / 32: 100003 rows, k = 512 0.52 / 0.55, 1024 0.76 /
+// 0.84, 1536 0.95 / 1.13, 2048 1.11 / 1.18, 4096 1.25 / 1.34; 8191 rows, k = 512 0.84 /
+// 0.91, 1024 0.96 / 1.24; 4095 rows, k = 512 0.98 / 1.31), or, with one tile, few
+// activations and a long K, the streaming kernel (97 rows, k = 4096, m = 1 / 8 / 16:
+// pair 2.05 / 2.38 / 2.81 of the streaming kernel's time, 1.59 / 2.00 / 2.48 of this one's).
+// Other K: the streaming kernel up to one tile per compute unit (n = 3584, k =
+// 18944: 14-15 / 18-20 / 33 us at m = 1 / 8 / 32 against 38.7 / 59 / 134), and up to
+// two where K is long (n = 8192, pair / streaming time, m = 1 / 8 / 16 / 32: k = 640
+// 0.84 / 0.75 / 0.87 / 0.75, 1920 0.98 / 0.94 / 1.02 / 0.87, 2176 1.02 / 0.99 / 1.06 /
+// 0.91, 3712 1.35 / 1.25 / 1.17 / 1.03, 5120 1.14 / 1.01 / 1.14 / 1.04); at n = 10240,
+// k = 5120 16.2 / 20.4 / 35 against 16.2 / 18.0 / 28.3 us.  Else the pair kernel's
+// INT8 form with P = 4 pairs in flight (equal to or faster than 2 and 8).
+// RLK_TUNE_W8_CFG = 1, 2, 3 selects the pair kernel with P = 2, 4, 8, 4, 5, 6 the
+// K-slice kernel with (lines per slice, tiles in flight) = (4, 1), (4, 2), (2, 2),
+// and 7 the streaming kernel.
 template <int MT, int MODE>
 int dispatch_w8(const W4Args& a, hipStream_t s) {
   int st = kNoFit;
@@ -1298,10 +1342,15 @@ int dispatch_w8(const W4Args& a, hipStream_t s) {
     case 5: st = launch_kslice_w8<4, 2, MT, MODE>(a, s); break;
     case 6: st = launch_kslice_w8<2, 2, MT, MODE>(a, s); break;
     case 7: st = launch_stream<MODE>(a, s); break;
-    default:
-      st = launch_kslice_w8<4, 1, MT, MODE>(a, s);
-      if (st == kNoFit && (a.n + 15) / 16 <= 2 * compute_units()) st = launch_stream<MODE>(a, s);
+    default: {
+      const int tiles = (a.n + 15) / 16, cus = compute_units();
+      const bool kslice = tiles <= cus ? a.m > 8 || a.k < 2560
+                                         : a.k >= (tiles <= 2 * cus ? 1024 : a.m >= 8 ? 1536 : 2048);
+      if (a.n % 16 == 0 || kslice) st = launch_kslice_w8<4, 1, MT, MODE>(a, s);
+      if (st == kNoFit && (tiles <= cus || (tiles <= 2 * cus && a.k > (a.m <= 16 ? 2048 : 3200))))
+        st = launch_stream<MODE>(a, s);
       break;
+    }
   }
   if (st == kNoFit) st = launch_pairs<4, MT, MODE, true>(a, s);
   return st;

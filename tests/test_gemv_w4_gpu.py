@@ -293,3 +293,22 @@ def test_gemv_w4_stream_odd_scales(torch_cuda, n, k, g, m):
     got = run_gemv(torch, x, packed, s, o, g, f32=True)
     assert rel_max_err(got[:, -1], want[:, -1]) <= 1e-5
     assert rel_max_err(got, want) <= 1e-5
+
+
+@pytest.mark.parametrize("n,k,g,m", [(2048, 2048, 128, 9), (2046, 1536, 128, 16), (4098, 1152, 128, 9),
+                                     (8192, 2304, 128, 16), (8206, 640, 128, 17), (4112, 1024, 128, 4),
+                                     (4112, 3456, 384, 32), (8210, 1024, 64, 9), (12290, 896, 32, 17),
+                                     (12304, 1024, 32, 16), (16386, 512, 64, 17), (16400, 512, 32, 9),
+                                     (20480, 160, 32, 3)])
+def test_gemv_w4_default_policy_edges(torch_cuda, n, k, g, m):
+    """The default policy on both sides of its lines between the streaming, K-slice,
+    pair and slab kernels (256 compute units): one to four tiles per unit, the K
+    and row counts where it changes.  The reference's bound."""
+    torch = torch_cuda
+    say(f"gemv_w4 policy n={n} k={k} g={g} m={m}")
+    rng = np.random.default_rng(n + k + m)
+    packed, s, o, _ = int4_linear(rng, n, k, g, dense=False)
+    x = randn_f16(rng, (m, k))
+    bias = randn_f16(rng, (n,), 0.1)
+    got = run_gemv(torch, x, packed, s, o, g, bias, f32=True)
+    assert rel_max_err(got, oracle.gemv_w4a16(x, packed, s, o, g, bias)) <= 1e-4

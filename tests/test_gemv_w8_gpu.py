@@ -193,3 +193,23 @@ def test_gemv_w8_row_tails_fp32_error(torch_cuda, n, k, m):
     want = (x.astype(np.float64) @ q.T.astype(np.float64)) * s.astype(np.float64)
     got = run_w8(torch_cuda, x, q, s, None, True).astype(np.float64)
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("n,k,m", [(97, 2560, 8), (97, 2560, 9), (97, 2048, 1), (4097, 512, 9), (4097, 1024, 9),
+                                   (8193, 1024, 8), (8193, 1536, 7), (8193, 1536, 8), (4112, 1920, 1),
+                                   (4112, 2176, 16), (4098, 2176, 17), (8192, 3328, 17), (8208, 3328, 17)])
+def test_gemv_w8_default_policy_edges(torch_cuda, n, k, m):
+    """The default policy on both sides of its lines between the K-slice, streaming
+    and pair kernels (256 compute units), with rows that fill tiles and that do
+    not.  fp32 at the reference's bound, exact codes (rows in part of a tile, or K
+    no multiple of 512) at 1e-6 of the result as in the test of the row tails."""
+    say(f"gemv_w8 policy n={n} k={k} m={m}")
+    rng = np.random.default_rng(n + k + m)
+    q = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    s = rng.uniform(0.001, 0.01, n).astype(np.float16)
+    x = randn_f16(rng, (m, k))
+    want = (x.astype(np.float64) @ q.T.astype(np.float64)) * s.astype(np.float64)
+    got = run_w8(torch_cuda, x, q, s, None, True).astype(np.float64)
+    assert rel_max_err(got, want) <= 1e-4
+    if n % 16 != 0 or k % 512 != 0:
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
