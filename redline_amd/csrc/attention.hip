@@ -1188,10 +1188,12 @@ bool launch_d(const AttnArgs& a, int G, bool int8, hipStream_t stream) {
   }
   if (a.w.max_partitions > 1) {
     // One thread group requests 32 rows in two batches, and 8 a round trip after
-    // that: past 32 partitions four groups share them (4 items x 28 heads of up to
-    // 128 partitions: the call 31.6 -> 29.9 us, one 32768-key item x 32 heads 35.5 -> 33.3).
+    // that; four groups share the rows but take about 1 us more to start and meet.
+    // They pay from about 50 partitions on: calls of 33 and 40 lose 0.7-1.2 us by
+    // them (64 items x 28 heads to 8300 keys 7 us), calls of 63 gain 0.3-2.3 where
+    // the contexts fill them, calls of 125 1.4-3.6.
     const dim3 grid(a.w.num_items, a.p.num_heads);
-    const bool wide = a.w.max_partitions > 32;
+    const bool wide = a.w.max_partitions > 48;
     if (runs) {
       if (wide) decode_reduce_kernel<D, true, 4><<<grid, 4 * D, 0, stream>>>(a);
       else decode_reduce_kernel<D, true, 1><<<grid, D, 0, stream>>>(a);

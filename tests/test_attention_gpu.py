@@ -199,10 +199,15 @@ LONG_CASES = {
     # splitting items: 2 to 157 partitions per item
     "runs": [40000, 9000, 300, 25000, 513, 17000, 4097, 30001, 257, 12000, 33000, 768,
              21000, 6000, 39000, 1100],
+    # the most partitions one thread group merges (48, 41, 34, 2 and 32 of them),
+    # and the fewest that four share
+    "48": [12288, 10241, 8449, 257, 8192],
+    "49": [12289, 8192, 12288, 300],
 }
 
 
-@pytest.mark.parametrize("lens,D", [("few", 64), ("few", 128), ("runs", 64), ("runs", 128)])
+@pytest.mark.parametrize("lens,D", [("few", 64), ("few", 128), ("runs", 64), ("runs", 128),
+                                    ("48", 128), ("49", 64)])
 @pytest.mark.parametrize("int8", [False, True])
 def test_decode_attention_long_contexts(torch_cuda, D, int8, lens, attention_form):
     """Long contexts (LONG_CASES), random cache contents."""
