@@ -68,8 +68,9 @@ struct PrefillArgs {
   rlk_attention_params p;
   rlk_prefill_attention_work w;
   int scale16;  // INT8 scales stored as fp16 (extension)
-  // ping-pong kernel: query heads per kv head, its reciprocal, kv heads x split = gridDim.x
-  int grp, split;
+  // ping-pong kernel: query heads per kv head, kv heads x split = gridDim.x (split a
+  // power of two, of the sequences or of their tiles), reciprocals
+  int grp, split, by_seq;
   float inv_grp, inv_hkv;
 };
 
@@ -987,18 +988,28 @@ __global__ __launch_bounds__(512, 2) void prefill_pp_kernel(PrefillArgs a) {
   const rlk_prefill_attention_work& w = a.w;
   // Sequences in reverse dispatch order and their last query tiles (the most
   // keys) first: in a chunked-prefill batch the later chunks usually sit deeper
-  // in their sequences, so the longest workgroups start first.  gridDim.x is a
-  // multiple of 8, so blockIdx.x picks the XCD: one kv head (and every
-  // gridDim.x / hkv-th query tile) of every sequence, which shares K and V in
-  // that XCD's L2 and gives each XCD the same work whatever the sequences'
-  // lengths.
+  // in their sequences, so the longest workgroups start first.  gridDim.x, kv
+  // heads x split, is a multiple of 8, so blockIdx.x picks the XCD: one kv head,
+  // which shares K and V in that XCD's L2, and one slot of the split.  Workgroups
+  // go to the XCDs in turn and a full one holds up the others, so the eight that
+  // follow each other should be alike, and no slot may stay empty:
+  //   by_seq (as many sequences as tiles): a slot takes every split-th sequence,
+  //     with all its tiles;
+  //   else: a slot takes every split-th tile of each sequence, from one that
+  //     turns with the sequence (a short one leaves slots without a tile).
+  // (176 prompts of 1661 tokens, 2 kv heads of 64, us: tiles without the turn 813,
+  // with it 665, by sequence 413; the kernel above 475.  4 kv heads, 4 prompts of 349
+  // .. 1748 tokens: tiles 54, by sequence 77.)
   const int hkv = p.kv.num_kv_heads, grp = a.grp;
-  const int sub = uniform_quot(blockIdx.x, a.inv_hkv), kvh = blockIdx.x - sub * hkv;
-  const int seq = w.seq_ids[gridDim.z - 1 - blockIdx.z];
+  const int slot = uniform_quot(blockIdx.x, a.inv_hkv), kvh = blockIdx.x - slot * hkv;
+  const int bz = blockIdx.z, nth_seq = a.by_seq ? bz * a.split + slot : bz;
+  if (nth_seq >= w.num_seqs) return;  // workgroup-uniform
+  const int seq = w.seq_ids[w.num_seqs - 1 - nth_seq];
   const int q_len = w.q_len[seq];
   const int nrows = q_len * grp;  // (token, head) rows of this kv head
   const int tile0 = (nrows + G::kBQ - 1) / G::kBQ - 1;  // the last tile
-  const int qrow0 = (tile0 - static_cast<int>(blockIdx.y) * a.split - sub) * G::kBQ;
+  const int nth_tile = a.by_seq ? blockIdx.y : blockIdx.y * a.split + ((slot + bz) & (a.split - 1));
+  const int qrow0 = (tile0 - nth_tile) * G::kBQ;
   if (qrow0 < 0) return;  // workgroup-uniform
   const int q0 = w.q_start[seq], past = w.ctx_len[seq] - q_len;
   const int lbs = __builtin_ctz(p.kv.block_size), bs = 1 << lbs;
@@ -1345,6 +1356,52 @@ int device_cus() {
   return cus[dev];
 }
 
+// Whether a call goes to the ping-pong kernel rather than the load-to-LDS one:
+// num_seqs sequences of up to `rows` tokens, tiles workgroups of 256 (token, head)
+// rows per kv head.  It needs the chip about half full (its workgroups start
+// later, 4-5 us, and take a whole compute unit: Llama heads, one prompt of 512 /
+// 1024 / 2048 tokens, 64 / 128 / 256 workgroups: 20.6 / 33.0 / 60.3 against 17.3 /
+// 30.3 / 99.6 us), and then wins by sharing K and V between the heads of a group
+// and filling rows that the other leaves empty.  Over 3000 drawn calls the
+// choice is 1.20 times as fast as the load-to-LDS kernel in the geometric mean and more
+// than 5% slower in 31 (at worst 18.0 against 13.0 us: 107 prompts of 52 .. 264 tokens,
+// one head).  Its exceptions, with that kernel's time over this one's:
+//   * one head per kv head: nothing is shared, and a short prompt leaves waves
+//     without rows.  D = 64: 17-64 tokens 0.6-1.1, 257-512 0.8-1.1 (FP16), 0.9-1.1
+//     (INT8), 513-1024 0.77-1.2 (FP16), 0.7-1.6 and 1.15 in the mean (INT8), past 1024
+//     1.0-1.7.  D = 128: up to 128 tokens 0.82-1.1 (FP16), 0.9-1.1 and from 512
+//     workgroups on 1.07-1.3 (INT8).
+//   * D = 64, 65-128 tokens: a whole 128-row workgroup of the other kernel.  This
+//     one's must be a sixth fewer rows (otherwise 0.79-1.1; with them 1.1-1.3).
+//   * FP16, several prompts of more than a tile: shorter ones than the longest
+//     leave workgroups empty (129-160 by count 0.81-1.3).
+bool ping_pong_pays(const rlk_attention_params& p, int num_seqs, int rows, int tiles) {
+  const int hkv = p.kv.num_kv_heads, grp = p.num_heads / hkv, cus = device_cus();
+  const bool int8 = p.kv.dtype == RLK_KV_INT8;
+  const int64_t wgs = static_cast<int64_t>(tiles) * hkv * num_seqs;
+  if (2 * wgs <= cus) return false;
+  if (grp == 1 && p.kv.head_dim == 64) return rows > (int8 ? 512 : 1024);
+  if (grp == 1 && rows <= 128) return int8 && wgs >= 2 * cus;
+  if (grp == 1) return true;
+  if (p.kv.head_dim == 64 && rows > 64 && rows <= 128) return 6 * 256 * tiles <= 5 * 128 * grp;
+  return int8 || num_seqs == 1 || tiles == 1 || 8 * wgs > 5 * cus;
+}
+
+// The same against the register-staged kernel, for calls the load-to-LDS kernel
+// cannot take (block tables past its LDS copy).  That one's workgroups start
+// soonest (one prompt of 38 tokens, Qwen2 heads, INT8: 6.9 against 12.1 us), but it
+// is the slowest over long prompts.  Its time over this kernel's, 240 drawn calls:
+// FP16, one head per kv head 0.92-2.1; groups, up to 256 tokens in at most 64
+// workgroups 0.64-1.5, in more 0.94-2; more tokens 1.0-2.6.  INT8, up to 512
+// tokens: one head per kv head 0.52-1.4, groups in at most 128 workgroups 0.57-1.3,
+// in more 0.91-1.5; past 512 tokens 0.96-1.6 (0.71 once).
+bool ping_pong_pays_wide(const rlk_attention_params& p, int num_seqs, int rows, int tiles) {
+  const int hkv = p.kv.num_kv_heads, grp = p.num_heads / hkv, cus = device_cus();
+  const int64_t wgs = static_cast<int64_t>(tiles) * hkv * num_seqs;
+  if (p.kv.dtype == RLK_KV_INT8) return rows > 512 || (grp > 1 && 2 * wgs > cus);
+  return grp == 1 || rows > 256 || 4 * wgs > cus;
+}
+
 int prefill(const rlk_attention_params* params, const rlk_prefill_attention_work* work,
             int scale16, hipStream_t stream) {
   const char* what = "paged_attention_prefill";
@@ -1392,20 +1449,18 @@ int prefill(const rlk_attention_params* params, const rlk_prefill_attention_work
   const bool dma_ok = dma_fits && (!int8 || !scale16 || p.kv.block_size % 2 == 0);
   // The ping-pong kernel: a wave's loads stay in one cache block (a power of
   // two of at least 8 rows); (token, head) rows and the cells of a block are
-  // counted in 32 bits (rows below 2^21: quot).  With fewer workgroups than
-  // half the compute units the kernel above is the faster one: its
-  // workgroups of 128 rows and one head are twice as many and start sooner (Llama
-  // heads, one prompt of 512 / 1024 / 2048 tokens, 64 / 128 / 256 workgroups:
-  // 20.6 / 33.0 / 60.3 against 17.3 / 30.3 / 99.6 us).
-  // RLK_TUNE_PREFILL_DMA = 2 forces this kernel, 1 the rule, 0 the register-staged one.
+  // counted in 32 bits (rows below 2^21: quot).  RLK_TUNE_PREFILL_DMA = 1 is the
+  // rule; 2 forces this kernel, 3 the load-to-LDS kernel where it can run, 0 the
+  // register-staged one.
   a.grp = p.num_heads / p.kv.num_kv_heads;
   const int pp_tiles = static_cast<int>((static_cast<int64_t>(rows) * a.grp + 255) / 256);
   const bool pp_ok = p.kv.block_size >= 8 && (p.kv.block_size & (p.kv.block_size - 1)) == 0 &&
                      static_cast<int64_t>(rows) * a.grp < (int64_t{1} << 21) && pp_tiles <= 65535 &&
                      static_cast<int64_t>(p.kv.num_kv_heads) * p.kv.block_size < (int64_t{1} << 30);
   const int path = tune_knob(kPrefillDma, 1);
-  const bool pp_fills = !dma_ok || 2 * static_cast<int64_t>(pp_tiles) * p.kv.num_kv_heads * w.num_seqs > device_cus();
-  if (pp_ok && (path >= 2 || (path == 1 && pp_fills))) {
+  const bool pays = dma_ok ? ping_pong_pays(p, w.num_seqs, rows, pp_tiles)
+                           : ping_pong_pays_wide(p, w.num_seqs, rows, pp_tiles);
+  if (pp_ok && (path == 2 || (path == 1 && pays))) {
     auto pp = [&](auto kernel, auto geo) -> int {
       using G = decltype(geo);
       const hipError_t e = grant_dynamic_lds(reinterpret_cast<const void*>(kernel), G::kLds);
@@ -1415,7 +1470,9 @@ int prefill(const rlk_attention_params* params, const rlk_prefill_attention_work
       while (p.kv.num_kv_heads * a.split % 8 != 0) a.split *= 2;
       a.inv_grp = 1.0f / static_cast<float>(a.grp);
       a.inv_hkv = 1.0f / static_cast<float>(p.kv.num_kv_heads);
-      const dim3 grid(p.kv.num_kv_heads * a.split, (pp_tiles + a.split - 1) / a.split, w.num_seqs);
+      a.by_seq = w.num_seqs >= std::max(a.split, pp_tiles);
+      const dim3 grid(p.kv.num_kv_heads * a.split, a.by_seq ? pp_tiles : (pp_tiles + a.split - 1) / a.split,
+                      a.by_seq ? (w.num_seqs + a.split - 1) / a.split : w.num_seqs);
       kernel<<<grid, G::kThreads, G::kLds, stream>>>(a);
       return launch_status(what);
     };
@@ -1429,7 +1486,7 @@ int prefill(const rlk_attention_params* params, const rlk_prefill_attention_work
     if (kv == kPfInt8F32) return pp(prefill_pp_kernel<128, kPfInt8F32>, PfPP<128, true>{});
     return pp(prefill_pp_kernel<128, kPfInt8F16>, PfPP<128, true>{});
   }
-  if (dma_ok && tune_knob(kPrefillDma, 1) != 0) {
+  if (dma_ok && path != 0) {
     auto dma = [&](auto kernel, auto geo) -> int {
       using G = decltype(geo);
       const size_t lds = G::lds_bytes(p.max_blocks_per_seq);

@@ -16,11 +16,16 @@ rows gathered into a compact buffer.  Larger cases cover several 64-row query
 tiles and 64-key tiles, contexts that are not multiples of either, fp16-stored
 INT8 scales, and the Llama-3.1-8B C3 chunks at full size (sampled rows).
 
-Prefill attention has two kernels: one that copies tiles to LDS with load-to-LDS
-instructions (the default when the block table fits its LDS copy) and one that
-stages them through registers (RLK_TUNE_PREFILL_DMA=0).  At D = 128 the first
-gives each wave 32 query rows, or 16 for small grids (RLK_TUNE_PREFILL_QS=1).
-Each test runs under the three settings."""
+Prefill attention has three kernels: the ping-pong kernel (block sizes that are a
+power of two; grids that fill the chip), one that copies tiles to LDS with
+load-to-LDS instructions (other grids, where the block table fits its LDS copy)
+and one that stages them through registers.  Each test runs with each of them
+forced (RLK_TUNE_PREFILL_DMA = 2, 3 and 0; a kernel that cannot take the call
+leaves it to the next), the load-to-LDS kernel at D = 128 with 32 query rows per
+wave and, as for small grids, 16 (RLK_TUNE_PREFILL_QS=1).  The ping-pong kernel's
+own cases, and the rule between the kernels, are in test_prefill_ping_pong_gpu.py."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -35,10 +40,10 @@ REF_CASES = [(8, 2, 128, False, [37, 300, 5]), (4, 4, 64, False, [64, 129, 1]),
              (8, 2, 128, True, [33, 280]), (4, 2, 64, True, [520])]
 
 
-@pytest.fixture(autouse=True, params=["dma", "dma16", "reg"])
+@pytest.fixture(autouse=True, params=["dma", "dma16", "reg", "pp"])
 def kernel_path(request):
     from redline_amd._lib import tune_knob
-    with tune_knob("RLK_TUNE_PREFILL_DMA", 0 if request.param == "reg" else 1), \
+    with tune_knob("RLK_TUNE_PREFILL_DMA", {"reg": 0, "pp": 2}.get(request.param, 3)), \
             tune_knob("RLK_TUNE_PREFILL_QS", 1 if request.param == "dma16" else 2):
         yield request.param
 
@@ -151,18 +156,9 @@ def test_prefill_attention_reference_geometries(torch_cuda, hq, hkv, D, int8, le
     assert_close_f16(got3, want[rows], what="chunked prefill")
 
 
-@pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("kv", ["fp16", "int8", "int8_f16scale"])
-@pytest.mark.parametrize("bs,pad", [(16, 0), (7, 0), (16, 4100)])
-def test_prefill_attention_random_cache_many_tiles(torch_cuda, D, kv, bs, pad, kernel_path):
-    """Several query and key tiles per sequence, GQA 4, random cache contents,
-    chunks with and without cached context (lengths not multiples of 64).
-    Block size 7 puts block boundaries at odd keys inside a tile; a block
-    table padded past 4096 columns exceeds the load-to-LDS kernel's LDS copy
-    of it (the register-staged kernel runs)."""
-    torch = torch_cuda
-    from redline_amd import kernels as K
-    say(f"prefill random D={D} kv={kv} bs={bs} pad={pad} path={kernel_path}")
+@functools.lru_cache(maxsize=None)
+def many_tiles_case(D, kv, bs):
+    """Inputs and the oracle's output (once for all kernels: seconds each)."""
     rng = np.random.default_rng(D + len(kv) + bs)
     hq, hkv = 8, 2
     int8 = kv != "fp16"
@@ -171,7 +167,7 @@ def test_prefill_attention_random_cache_many_tiles(torch_cuda, D, kv, bs, pad, k
     S = len(chunks)
     nblk = 1 + sum((L + bs - 1) // bs for L in lens)
     ids = rng.permutation(np.arange(1, nblk)).astype(np.int32)
-    maxb = max((L + bs - 1) // bs for L in lens) + pad
+    maxb = max((L + bs - 1) // bs for L in lens)
     tables = np.zeros((S, maxb), np.int32)
     nxt = 0
     for i, L in enumerate(lens):
@@ -195,10 +191,30 @@ def test_prefill_attention_random_cache_many_tiles(torch_cuda, D, kv, bs, pad, k
     ctx = np.array(lens, np.int32)
     T = int(q_len.sum())
     q = randn_f16(rng, (T, hq * D))
-    scale = 1 / np.sqrt(D)
     sid = np.arange(S, dtype=np.int32)
-    want = oracle.paged_attention_prefill(q, hq * D, hq, scale, kc, vc, kscl, vscl, tables, sid,
+    want = oracle.paged_attention_prefill(q, hq * D, hq, 1 / np.sqrt(D), kc, vc, kscl, vscl, tables, sid,
                                           q_start, q_len, ctx, T, int8)
+    return hq, hkv, nblk, tables, kc, vc, kscl, vscl, q, sid, q_start, q_len, ctx, want
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("kv", ["fp16", "int8", "int8_f16scale"])
+@pytest.mark.parametrize("bs,pad", [(16, 0), (7, 0), (16, 4100)])
+def test_prefill_attention_random_cache_many_tiles(torch_cuda, D, kv, bs, pad, kernel_path):
+    """Several query and key tiles per sequence, GQA 4, random cache contents,
+    chunks with and without cached context (lengths not multiples of 64).
+    Block size 7 puts block boundaries at odd keys inside a tile; a block
+    table padded past 4096 columns exceeds the load-to-LDS kernel's LDS copy
+    of it (the register-staged kernel runs there, or the ping-pong kernel, which
+    reads the table in place)."""
+    torch = torch_cuda
+    from redline_amd import kernels as K
+    say(f"prefill random D={D} kv={kv} bs={bs} pad={pad} path={kernel_path}")
+    int8 = kv != "fp16"
+    hq, hkv, nblk, tables, kc, vc, kscl, vscl, q, sid, q_start, q_len, ctx, want = many_tiles_case(D, kv, bs)
+    tables = np.pad(tables, ((0, 0), (0, pad)))
+    S, maxb = tables.shape
+    T, scale = len(q), 1 / np.sqrt(D)
 
     cache = K.KVCache(1, nblk, hkv, D, bs, K.KVDType.kINT8 if int8 else K.KVDType.kFP16)
     k, v, ksc, vsc = cache.tensors(0)
@@ -381,63 +397,3 @@ def test_prefill_attention_full_chip_repeats(torch_cuda, int8):
         s = (q[-n:, h * D:(h + 1) * D].float() @ k[:, h // (hq // hkv)].t().contiguous()) * D ** -0.5
         want = torch.softmax(s.masked_fill(mask, float("-inf")), -1) @ v[:, h // (hq // hkv)].contiguous()
         assert_close_f16(got[0][-n:, h * D:(h + 1) * D], want.cpu().numpy(), what=f"head {h}")
-
-
-@pytest.mark.parametrize("D,kv", [(64, "fp16"), (128, "fp16"), (64, "int8"), (128, "int8"),
-                                  (64, "int8_f16scale"), (128, "int8_f16scale")])
-@pytest.mark.parametrize("bs,hq,hkv", [(8, 7, 1), (16, 8, 8), (16, 28, 4), (32, 24, 3), (128, 16, 2)])
-def test_prefill_attention_ping_pong(torch_cuda, D, kv, bs, hq, hkv, kernel_path):
-    """The ping-pong kernel, forced at small grids: (token, head) rows that fill
-    workgroups only in part and straddle them, one tile of keys and many, tile
-    ends on and off 64 keys, blocks smaller and larger than a tile, kv heads that
-    do and do not divide the XCDs; against fp32 torch attention over the cache
-    (INT8: through fp16, as the kernel contract has it).  Written output rows only."""
-    if kernel_path != "dma":
-        pytest.skip("one kernel: the paths of this module do not apply")
-    torch = torch_cuda
-    from redline_amd import kernels as K
-    from redline_amd._lib import tune_knob
-    say(f"prefill ping-pong D={D} kv={kv} bs={bs} hq={hq} hkv={hkv}")
-    segs = [(0, 2), (63, 2), (0, 64), (64, 65), (200, 300), (0, 33), (447, 65), (5, 130)]
-    rng = np.random.default_rng(D + bs + hq)
-    g = torch.Generator(device="cuda").manual_seed(D + bs + hq)
-    need = [(s + n + bs - 1) // bs for s, n in segs]
-    S, T, G = len(segs), sum(n for _, n in segs), hq // hkv
-    cache = K.KVCache(1, sum(need) + 1, hkv, D, bs, K.KVDType.kFP16 if kv == "fp16" else K.KVDType.kINT8,
-                      scale_dtype=K.SCALE_F16 if kv == "int8_f16scale" else K.SCALE_F32)
-    for i, t in enumerate(x for x in cache.tensors(0) if x is not None):
-        if t.dtype == torch.int8:
-            t.copy_(torch.randint(-127, 128, t.shape, generator=g, device="cuda", dtype=torch.int8))
-        elif i < 2:
-            t.normal_(generator=g)
-        else:
-            t.uniform_(0.008, 0.018, generator=g)
-    pool = rng.permutation(np.arange(1, sum(need) + 1, dtype=np.int32))
-    bb = ra.BatchBuilder(T, S, S, max(need), bs, 1)
-    tables, at = [], 0
-    for (s, n), k in zip(segs, need):
-        tables.append(pool[at:at + k])
-        bb.add(np.zeros(n, np.int32), s, n, None, pool[at:at + k])
-        at += k
-    meta, shape, lay = bb.write()
-    d_meta = dev(torch, meta)
-    stride = (hq + 2 * hkv) * D
-    q = (1.5 * torch.randn((T, stride), generator=g, device="cuda")).half()
-    with tune_knob("RLK_TUNE_PREFILL_DMA", 2):
-        got = run_prefill(torch, K, q, stride, hq, D ** -0.5, cache.layer(0), d_meta[lay["block_tables"]:],
-                          max(need), d_meta[lay["positions"]:], d_meta, lay, shape, T, D,
-                          scale16=kv == "int8_f16scale")
-    k, v, ks, vs = cache.tensors(0)
-    at = 0
-    for (s, n), t in zip(segs, tables):
-        idx = torch.from_numpy(t.astype(np.int64)).cuda()
-        rows = lambda x, sc: (x[idx].float() if sc is None else  # noqa: E731
-                              (x[idx].float() * sc[idx].float()[..., None]).half().float()
-                              ).transpose(1, 2).reshape(-1, hkv, D)[:s + n]
-        kk, vv = rows(k, ks), rows(v, vs)
-        mask = torch.arange(s + n, device="cuda")[None] > s + torch.arange(n, device="cuda")[:, None]
-        for h in range(hq):
-            sc = (q[at:at + n, h * D:(h + 1) * D].float() @ kk[:, h // G].t().contiguous()) * D ** -0.5
-            want = torch.softmax(sc.masked_fill(mask, float("-inf")), -1) @ vv[:, h // G].contiguous()
-            assert_close_f16(got[at:at + n, h * D:(h + 1) * D], want.cpu().numpy(), what=f"segment {s}+{n} head {h}")
-        at += n
