@@ -851,15 +851,18 @@ __global__ __launch_bounds__((64 * kslice_max_waves<CPW, MT>())) void gemv_w4_ks
 // per 8 codes, int8x8_to_f16_biased); each tile's sum starts from -1152
 // sum(x) of the slice, so the products leave x . code.  The row scale and
 // the bias apply once, to the reduced sum (gemv_weight_only.cu:36).
-// kTail: n may end inside a tile, and the codes are exact (4 VALU more per 8
+// kRowsTail: n may end inside a tile, and the codes are exact (4 VALU more per 8
 // codes): the bias costs fp32 sum bits (2.5e-6 of the result at K = 4096 against
 // 4e-7), which products of such n, the pair kernel's otherwise, do not give up.
-template <int CPW, int U, int MT, int MODE, bool kTail>
+// kRowsClamped: whole tiles, with the tail form's clamped row offsets, which change
+// nothing but the schedule of the loads: better with 4 waves and more (28672 x 4096,
+// m = 1 / 32: 21.8 / 24.3 us with, 22.3 / 25.3 without), worse with fewer (65536 x 1024:
+// 17.9 / 22.3 against 17.4 / 21.3).
+enum KsliceRows { kRowsWhole, kRowsClamped, kRowsTail };
+template <int CPW, int U, int MT, int MODE, KsliceRows ROWS>
 __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a) {
   constexpr int P = CPW * U;  // ring depth in lines: U tiles
-  // (clamped row offsets are part of the schedule with two activation tiles: 28672 x
-  // 4096, m = 32: 25.1 us with, 26.1 without; with one tile 65536 x 1024: 17.9 / 17.4)
-  constexpr bool kClamp = kTail || MT == 2;
+  constexpr bool kTail = ROWS == kRowsTail, kClamp = ROWS != kRowsWhole;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int threads = blockDim.x, nw = threads / 64;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -867,7 +870,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
   const int r16 = lane & 15, qd = lane >> 4;
   const bool low = (lane & 8) == 0;
   const int T = a.cpp;  // tiles per workgroup, a multiple of U
-  const int ntiles = kTail ? (a.n + 15) / 16 : a.n / 16;
+  const int ntiles = kClamp ? (a.n + 15) / 16 : a.n / 16;
   const int tile0 = blockIdx.x * T;
   f32x4* red = reinterpret_cast<f32x4*>(lds);  // [T][nw][MT][64 lanes]
   const int kb = a.k;
@@ -970,7 +973,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w8_kslice_kernel(W4Args a
   for (int t = wave; t < T; t += nw) {
     const int row = (tile0 + t) * 16 + r16;
     if (tile0 + t >= ntiles) break;
-    const float sc = static_cast<float>(__builtin_bit_cast(_Float16, a.scales[kTail ? min(row, a.n - 1) : row]));
+    const float sc = static_cast<float>(__builtin_bit_cast(_Float16, a.scales[kClamp ? min(row, a.n - 1) : row]));
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       f32x4 sum = red[((t * nw) * MT + mt) * kWave + lane];
@@ -1298,8 +1301,9 @@ int launch_kslice_w8(W4Args a, hipStream_t stream) {
   if (lds_for(T) > kLdsBudget) return kNoFit;
   a.cpp = T;
   const size_t lds = lds_for(T);
-  auto kernel = a.n % 16 == 0 ? gemv_w8_kslice_kernel<CPW, U, MT, MODE, false>
-                              : gemv_w8_kslice_kernel<CPW, U, MT, MODE, true>;
+  auto kernel = a.n % 16 != 0 ? gemv_w8_kslice_kernel<CPW, U, MT, MODE, kRowsTail>
+                : nw >= 4     ? gemv_w8_kslice_kernel<CPW, U, MT, MODE, kRowsClamped>
+                              : gemv_w8_kslice_kernel<CPW, U, MT, MODE, kRowsWhole>;
   if (lds > 64 * 1024) {
     const hipError_t e = grant_dynamic_lds(reinterpret_cast<const void*>(kernel), kLdsBudget);
     if (e != hipSuccess)
