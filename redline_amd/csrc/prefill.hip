@@ -68,9 +68,10 @@ struct PrefillArgs {
   rlk_attention_params p;
   rlk_prefill_attention_work w;
   int scale16;  // INT8 scales stored as fp16 (extension)
-  // ping-pong kernel: query heads per kv head, kv heads x split = gridDim.x (split a
-  // power of two, of the sequences or of their tiles), reciprocals
-  int grp, split, by_seq;
+  // ping-pong kernel: query heads per kv head; kv heads x split = gridDim.x, the split
+  // (a power of two) of the sequences (by_seq: seq_step = split, tile_step = 1) or of
+  // their tiles (0: seq_step = 1, tile_step = split); reciprocals
+  int grp, by_seq, seq_step, tile_step, last_seq;
   float inv_grp, inv_hkv;
 };
 
@@ -1002,13 +1003,14 @@ __global__ __launch_bounds__(512, 2) void prefill_pp_kernel(PrefillArgs a) {
   // .. 1748 tokens: tiles 54, by sequence 77.)
   const int hkv = p.kv.num_kv_heads, grp = a.grp;
   const int slot = uniform_quot(blockIdx.x, a.inv_hkv), kvh = blockIdx.x - slot * hkv;
-  const int bz = blockIdx.z, nth_seq = a.by_seq ? bz * a.split + slot : bz;
-  if (nth_seq >= w.num_seqs) return;  // workgroup-uniform
-  const int seq = w.seq_ids[w.num_seqs - 1 - nth_seq];
-  const int q_len = w.q_len[seq];
+  const int nth_seq = a.last_seq - static_cast<int>(blockIdx.z) * a.seq_step - slot * a.by_seq;
+  // (past the first sequence: no rows.  A return here would put the loads below
+  // after its wait: 0.9% of the 4 x 4096-token INT8 call)
+  const int seq = w.seq_ids[max(nth_seq, 0)];
+  const int q_len = nth_seq < 0 ? 0 : w.q_len[seq];
   const int nrows = q_len * grp;  // (token, head) rows of this kv head
   const int tile0 = (nrows + G::kBQ - 1) / G::kBQ - 1;  // the last tile
-  const int nth_tile = a.by_seq ? blockIdx.y : blockIdx.y * a.split + ((slot + bz) & (a.split - 1));
+  const int nth_tile = static_cast<int>(blockIdx.y) * a.tile_step + ((slot + blockIdx.z) & (a.tile_step - 1));
   const int qrow0 = (tile0 - nth_tile) * G::kBQ;
   if (qrow0 < 0) return;  // workgroup-uniform
   const int q0 = w.q_start[seq], past = w.ctx_len[seq] - q_len;
@@ -1466,13 +1468,16 @@ int prefill(const rlk_attention_params* params, const rlk_prefill_attention_work
       const hipError_t e = grant_dynamic_lds(reinterpret_cast<const void*>(kernel), G::kLds);
       if (e != hipSuccess)
         return fail(RLK_EUNSUPPORTED, "%s: %d bytes of LDS refused (%s)", what, G::kLds, hipGetErrorString(e));
-      a.split = 1;  // kv heads x split: a multiple of the 8 XCDs
-      while (p.kv.num_kv_heads * a.split % 8 != 0) a.split *= 2;
+      int split = 1;  // kv heads x split: a multiple of the 8 XCDs
+      while (p.kv.num_kv_heads * split % 8 != 0) split *= 2;
+      a.by_seq = w.num_seqs >= std::max(split, pp_tiles);
+      a.seq_step = a.by_seq ? split : 1;
+      a.tile_step = a.by_seq ? 1 : split;
+      a.last_seq = w.num_seqs - 1;
       a.inv_grp = 1.0f / static_cast<float>(a.grp);
       a.inv_hkv = 1.0f / static_cast<float>(p.kv.num_kv_heads);
-      a.by_seq = w.num_seqs >= std::max(a.split, pp_tiles);
-      const dim3 grid(p.kv.num_kv_heads * a.split, a.by_seq ? pp_tiles : (pp_tiles + a.split - 1) / a.split,
-                      a.by_seq ? (w.num_seqs + a.split - 1) / a.split : w.num_seqs);
+      const dim3 grid(p.kv.num_kv_heads * split, (pp_tiles + a.tile_step - 1) / a.tile_step,
+                      (w.num_seqs + a.seq_step - 1) / a.seq_step);
       kernel<<<grid, G::kThreads, G::kLds, stream>>>(a);
       return launch_status(what);
     };
