@@ -8,8 +8,7 @@ tests/cuda/test_gemm.cu:134-160) and fp16 outputs at fp16 tolerance.
 Geometries: the reference test's (n = 97, k = 512, m in 1, 3, 8, 13, 16, with a
 bias), K that is not a multiple of the 128-K chunk pair (16 .. 1040), m up to 32
 (two activation tiles), Llama-3.1-8B projections (gate: n = 14336, k = 4096;
-down: n = 4096, k = 14336, where x is staged in several passes) and every
-launch policy."""
+down: n = 4096, k = 14336) and every launch policy."""
 
 import numpy as np
 import pytest
@@ -48,7 +47,8 @@ def run_w8(torch, x, q, s, bias=None, f32=False):
 @pytest.mark.parametrize("f32", [True, False])
 @pytest.mark.parametrize("m", [1, 3, 8, 13, 16, 20, 32])
 def test_gemv_w8_reference_geometry(torch_cuda, m, f32):
-    """tests/cuda/test_gemm.cu:134-160: n = 97 (odd: the row tail), k = 512, bias."""
+    """tests/cuda/test_gemm.cu:134-160: n = 97 (odd: the row tail), k = 512, bias.
+    The default policy (the K-slice kernel), the pair and the streaming kernel."""
     say(f"gemv_w8 reference geometry m={m} f32={f32}")
     rng = np.random.default_rng(100 + m)
     n, k = 97, 512
@@ -56,11 +56,13 @@ def test_gemv_w8_reference_geometry(torch_cuda, m, f32):
     bias = randn_f16(rng, (n,), 0.02)
     x = randn_f16(rng, (m, k))
     want = oracle.gemv_w8a16(x, q, s, bias)
-    got = run_w8(torch_cuda, x, q, s, bias, f32)
-    if f32:
-        assert rel_max_err(got, want) <= 1e-4
-    else:
-        assert_close_f16(got, want, what="w8 f16")
+    for cfg in (None, 2, 7):
+        with tune_knob("RLK_TUNE_W8_CFG", cfg):
+            got = run_w8(torch_cuda, x, q, s, bias, f32)
+        if f32:
+            assert rel_max_err(got, want) <= 1e-4, cfg
+        else:
+            assert_close_f16(got, want, what=f"w8 f16 cfg={cfg}")
 
 
 @pytest.mark.parametrize("k", [16, 80, 144, 528, 1040])
@@ -81,18 +83,21 @@ def test_gemv_w8_k_not_a_whole_chunk_pair(torch_cuda, k, m):
 @pytest.mark.parametrize("n,k,m", [(14336, 4096, 1), (14336, 4096, 16), (4096, 14336, 4),
                                    (4096, 14336, 32)])
 def test_gemv_w8_llama_projections(torch_cuda, n, k, m):
-    """Llama-3.1-8B gate (n = 14336, k = 4096) and down (n = 4096, k = 14336;
-    x of 4 rows and more is staged in several passes)."""
+    """Llama-3.1-8B gate (n = 14336, k = 4096) and down (n = 4096, k = 14336),
+    by the default policy and by the pair kernel (2; x of 4 rows and more of the
+    down projection is staged in several passes)."""
     say(f"gemv_w8 llama n={n} k={k} m={m}")
     rng = np.random.default_rng(n + m)
     q, s, _ = int8_linear(rng, n, k, 0.02)
     x = randn_f16(rng, (m, k))
     want = oracle.gemv_w8a16(x, q, s)
-    got = run_w8(torch_cuda, x, q, s, None, False)
-    assert_close_f16(got, want, what="llama w8")
+    for cfg in (None, 2):
+        with tune_knob("RLK_TUNE_W8_CFG", cfg):
+            got = run_w8(torch_cuda, x, q, s, None, False)
+        assert_close_f16(got, want, what=f"llama w8 cfg={cfg}")
 
 
-@pytest.mark.parametrize("cfg", range(7))
+@pytest.mark.parametrize("cfg", range(8))
 def test_gemv_w8_launch_policies_agree(torch_cuda, cfg):
     say(f"gemv_w8 cfg={cfg}")
     rng = np.random.default_rng(cfg)
