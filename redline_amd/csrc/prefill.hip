@@ -911,7 +911,10 @@ prefill_dma_kernel(PrefillArgs a) {
 //   FP16: load-to-LDS of tile t + 3 in X(t).
 //   INT8: the codes (16 bytes of K and V a lane, 8 at D = 64) and the row's
 //     scales go to registers two tiles earlier; Y(t) dequantises tile t + 2 into
-//     its fp16 stage, fp16(float(code) * scale).
+//     its fp16 stage, fp16(float(code) * scale).  That distance holds for fp32
+//     scales only: the compiler packs the two fp16 scales into one register where
+//     they are loaded, which waits for all of the tile's loads inside X, and at
+//     D = 64 keeps the pair in scratch (48 bytes a lane).
 // 16-byte chunk c of row r lies at c ^ kswz(r) in a K tile and c ^ vswz(r) in a V
 // tile: the 16 rows of a K read then take 16 different slots of 256 bytes, and
 // the 4 rows x 64 bytes that 32 lanes of a transposing V read take fill them.
