@@ -164,7 +164,12 @@ __device__ __forceinline__ float row_bias(const W4Args& a, int row) {
 }
 template <int MODE>
 __device__ __forceinline__ void store_tile(const W4Args& a, f32x4 v, int m0, int row, int r16) {
-  store_tile<MODE>(a, v, row_bias(a, row), m0, row, r16);
+  if constexpr (MODE == kModeSwiglu) {
+    store_tile<MODE>(a, v, 0.f, m0, row, r16);
+  } else {
+    if (row >= a.n) return;
+    store_tile<MODE>(a, v, row_bias(a, row), m0, row, r16);
+  }
 }
 
 constexpr int kMaxWaves = 8;  // of a workgroup: two waves per SIMD, up to 256 VGPRs each
