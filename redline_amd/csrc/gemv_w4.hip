@@ -1314,23 +1314,45 @@ int launch_kslice_w8(W4Args a, hipStream_t stream) {
   return RLK_OK;
 }
 
+// Where n ends inside a tile: whether the K-slice kernel (exact codes there) or the
+// pair kernel, with one tile and a long K the streaming one.  The pair kernel has a wave per
+// tile of a compute unit, up to 8, each over the whole K: it is at its best with 4 to 8
+// tiles, which are one full round, and worst just past 8.  The K-slice kernel has
+// k / 512 waves for any number of tiles.  Pair / K-slice time, m = 1 / 8 / 16 / 32, by
+// tiles per compute unit:
+//   1: 97 rows, k = 4096, m = 1 / 8 / 16: pair 2.05 / 2.38 / 2.81 of the streaming kernel's
+//     time, 1.59 / 2.00 / 2.48 of this one's;
+//   2: k = 512 0.84 / - / - / 0.91, 1024 0.96 / - / - / 1.24;
+//   2.4: k = 1536 0.97 / 0.96 / 0.99 / 1.22, 2048 1.05 / 1.11 / 1.17 / 1.34;
+//   3.9: k = 1536 0.86 / 0.87 / 0.90 / 0.96, 2048 0.94 / 0.95 / 0.99 / 1.12, 3584 0.94 / 0.97 /
+//     1.06 / 1.34, 4096 1.03 / 1.07 / 1.17 / 1.44;
+//   6.8: k = 2048 0.96 / 0.97 / 0.99 / 1.00, 2560 0.93 / 0.93 / 0.95 / 1.12, 3584 0.96 / 0.97 / 1.01 /
+//     1.20, 4096 1.06 / 1.14 / 1.17 / 1.27;
+//   8.1: k = 1536 1.09 / 1.12 / 1.19 / 1.20, 2048 1.27 / 1.32 / 1.40 / 1.38;
+//   14: k = 1536 0.85 / 0.90 / 0.93 / 0.92, 2048 0.95 / 0.97 / 1.04 / 1.09;
+//   24: k = 512 0.52 / - / - / 0.55, 1024 0.76 / - / - / 0.84, 2048 1.07 / 1.10 / 1.14 / 1.16.
+bool kslice_tail_pays(int m, int k, int tiles, int cus) {
+  if (tiles <= cus) return m > 8 || k < 2560;
+  if (tiles <= 2 * cus) return k >= 1024;
+  if (tiles <= 3 * cus) return k >= 2048 || (k >= 1536 && m > 16);
+  if (tiles <= 8 * cus) return k >= 4096 || (m > 16 && (tiles <= 6 * cus ? k >= 2048 : k > 2048));
+  return k >= 2048 || (k >= 1536 && tiles <= 12 * cus);
+}
+
 // INT8 weight-only GEMV (gemv_weight_only.cu:64-93): the K-slice kernel with
 // one tile's lines in flight where it fits (K a multiple of 512 up to 4096: at
 // the Llama-3.1-8B gate_up shape 23.2 / 23.4 / 23.6 / 26.4 us at m = 1 / 8 /
 // 16 / 32 against 25.0 / 25.7 / 26.5 / 30.7 for the pair kernel, same run).
-// Where n ends inside a tile the other choice is the pair kernel, which a
-// workgroup of k / 512 waves only beats if it has enough of them for its tiles
-// (pair / K-slice time, m = 1 / 32: 100003 rows, k = 512 0.52 / 0.55, 1024 0.76 /
-// 0.84, 1536 0.95 / 1.13, 2048 1.11 / 1.18, 4096 1.25 / 1.34; 8191 rows, k = 512 0.84 /
-// 0.91, 1024 0.96 / 1.24; 4095 rows, k = 512 0.98 / 1.31), or, with one tile, few
-// activations and a long K, the streaming kernel (97 rows, k = 4096, m = 1 / 8 / 16:
-// pair 2.05 / 2.38 / 2.81 of the streaming kernel's time, 1.59 / 2.00 / 2.48 of this one's).
+// Where n ends inside a tile kslice_tail_pays has the say.
 // Other K: the streaming kernel up to one tile per compute unit (n = 3584, k =
 // 18944: 14-15 / 18-20 / 33 us at m = 1 / 8 / 32 against 38.7 / 59 / 134), and up to
 // two where K is long (n = 8192, pair / streaming time, m = 1 / 8 / 16 / 32: k = 640
 // 0.84 / 0.75 / 0.87 / 0.75, 1920 0.98 / 0.94 / 1.02 / 0.87, 2176 1.02 / 0.99 / 1.06 /
 // 0.91, 3712 1.35 / 1.25 / 1.17 / 1.03, 5120 1.14 / 1.01 / 1.14 / 1.04); at n = 10240,
-// k = 5120 16.2 / 20.4 / 35 against 16.2 / 18.0 / 28.3 us.  Else the pair kernel's
+// k = 5120 16.2 / 20.4 / 35 against 16.2 / 18.0 / 28.3 us.  Three steps of 128 codes
+// leave most of its eight waves without one: up to K = 384 the pair kernel (n = 16 .. 4096,
+// pair / streaming time, m = 1 / 8 / 17: k = 128 0.85-0.99 / 0.85-0.98 / 0.81-0.94, 384
+// 0.93-1.00 / 0.87-0.98 / 0.90-0.99; 640 0.98-1.03 / 0.95-1.03 / 0.99-1.05).  Else the pair kernel's
 // INT8 form with P = 4 pairs in flight (equal to or faster than 2 and 8).
 // RLK_TUNE_W8_CFG = 1, 2, 3 selects the pair kernel with P = 2, 4, 8, 4, 5, 6 the
 // K-slice kernel with (lines per slice, tiles in flight) = (4, 1), (4, 2), (2, 2),
@@ -1348,10 +1370,8 @@ int dispatch_w8(const W4Args& a, hipStream_t s) {
     case 7: st = launch_stream<MODE>(a, s); break;
     default: {
       const int tiles = (a.n + 15) / 16, cus = compute_units();
-      const bool kslice = tiles <= cus ? a.m > 8 || a.k < 2560
-                                         : a.k >= (tiles <= 2 * cus ? 1024 : a.m >= 8 ? 1536 : 2048);
-      if (a.n % 16 == 0 || kslice) st = launch_kslice_w8<4, 1, MT, MODE>(a, s);
-      if (st == kNoFit && (tiles <= cus || (tiles <= 2 * cus && a.k > (a.m <= 16 ? 2048 : 3200))))
+      if (a.n % 16 == 0 || kslice_tail_pays(a.m, a.k, tiles, cus)) st = launch_kslice_w8<4, 1, MT, MODE>(a, s);
+      if (st == kNoFit && a.k > 384 && (tiles <= cus || (tiles <= 2 * cus && a.k > (a.m <= 16 ? 2048 : 3200))))
         st = launch_stream<MODE>(a, s);
       break;
     }

@@ -202,7 +202,10 @@ def test_gemv_w8_row_tails_fp32_error(torch_cuda, n, k, m):
 
 @pytest.mark.parametrize("n,k,m", [(97, 2560, 8), (97, 2560, 9), (97, 2048, 1), (4097, 512, 9), (4097, 1024, 9),
                                    (8193, 1024, 8), (8193, 1536, 7), (8193, 1536, 8), (4112, 1920, 1),
-                                   (4112, 2176, 16), (4098, 2176, 17), (8192, 3328, 17), (8208, 3328, 17)])
+                                   (4112, 2176, 16), (4098, 2176, 17), (8192, 3328, 17), (8208, 3328, 17),
+                                   (97, 384, 8), (96, 640, 8), (8193, 1536, 16), (8193, 1536, 17), (12305, 2048, 16),
+                                   (12305, 2048, 17), (12305, 3584, 16), (12305, 4096, 1), (24593, 2048, 17),
+                                   (33009, 1536, 1), (49169, 1536, 1)])
 def test_gemv_w8_default_policy_edges(torch_cuda, n, k, m):
     """The default policy on both sides of its lines between the K-slice, streaming
     and pair kernels (256 compute units), with rows that fill tiles and that do
